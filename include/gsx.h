@@ -405,6 +405,28 @@ int gsx_raster_bwd(int64_t n, int32_t C, const float* means2d,
                    float* g_opacities, int32_t grad_stride,
                    int32_t* tile_order, void* stream);
 
+/* The same backward with the six geometric gradients in one record per
+ * Gaussian (g_geometry, 16-byte aligned, grad_stride >= 8 floats, a multiple of
+ * 4: [means2d 2 | conic 3 | opacity 1 | padding]) and the channels' in an array
+ * of their own (g_features (N,C)): one cache line for the geometric atomics
+ * instead of three arrays' lines, and a feature gradient the caller can hand on
+ * as it is.  gsx_preprocess_bwd without SH reads such a record in place;
+ * gsx_split_raster_grads writes its three parts as separate arrays. */
+int gsx_raster_bwd_geometry(int64_t n, int32_t C, const float* means2d,
+                            const float* conic_opacity, const float* features,
+                            const int32_t* sorted_ids, int64_t num_ids,
+                            const int32_t* tile_ranges,
+                            const float* background, int32_t width,
+                            int32_t height, const float* final_T,
+                            const int32_t* n_contrib, const float* grad_out,
+                            const float* grad_final_T, float* g_geometry,
+                            float* g_features, int32_t grad_stride,
+                            int32_t* tile_order, void* stream);
+
+int gsx_split_raster_grads(int64_t n, const float* record, int32_t grad_stride,
+                           float* g_means2d, float* g_conics,
+                           float* g_opacities, void* stream);
+
 /* -------------------------------------------------------- training step --
  * The calls GaussianTrainer.step (splatting/trainer.py:319-421) makes
  * around the render. */

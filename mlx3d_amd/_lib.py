@@ -148,6 +148,9 @@ SIGNATURES = {
     "gsx_tile_order_words": (_I64, [_I32, _I32]),
     "gsx_raster_bwd": (ctypes.c_int, [_I64, _I32, _P, _P, _P, _P, _I64, _P, _P, _I32, _I32, _P,
                                       _P, _P, _P, _P, _P, _P, _P, _I32, _P, _P]),
+    "gsx_raster_bwd_geometry": (ctypes.c_int, [_I64, _I32, _P, _P, _P, _P, _I64, _P, _P, _I32,
+                                               _I32, _P, _P, _P, _P, _P, _P, _I32, _P, _P]),
+    "gsx_split_raster_grads": (ctypes.c_int, [_I64, _P, _I32, _P, _P, _P, _P]),
     "gsx_photometric_workspace_bytes": (_I64, [_I32, _I32, _I32]),
     "gsx_photometric_fwd": (ctypes.c_int, [_I32, _I32, _I32, _P, _P, _I32, _F, _F, _P, _I64, _P,
                                            _P]),

@@ -20,14 +20,16 @@
 // below 1e-4), branch-free per pair; a wave stops once its 64 pixels have
 // terminated and the workgroup stops loading once all 256 have.
 // Backward: back-to-front replay (rasterize.py:147-220) from the largest
-// n_contrib of each quadrant.  A pair's gradient terms are summed over the
-// wave with cross-row swaps and DPP row operations (two Gaussians per
-// reduction up to four channels); lane 15 of each row stores its share of
-// the sums in the wave's own LDS slot for that Gaussian (no LDS atomics),
-// and after the batch one lane per Gaussian adds the four waves' slots and
-// issues one global atomic per (Gaussian, tile, component) -- the reference
-// issues one per (pixel, Gaussian, component).
+// n_contrib of each quadrant; the reference issues one atomic per (pixel,
+// Gaussian, component).  Up to four channels (k_raster_bwd) the lanes are
+// pixels: a pair's gradient terms are summed over the wave with cross-row
+// swaps and DPP row operations, two Gaussians per reduction, and after the
+// batch one lane per Gaussian adds the four waves' slots and issues one
+// global atomic per (Gaussian, tile, component).  From five channels on
+// (k_raster_bwd_wide) the lanes are Gaussians and the channel work runs on
+// the matrix cores.
 #include <algorithm>
+#include <type_traits>
 
 #include "gsx_device.h"
 #include "tile_order.h"
@@ -164,6 +166,27 @@ __device__ __forceinline__ uint32_t quadrant_mask(float x, float y, float4 c, in
            ((inl && inb) || q2 <= t2 ? 4u : 0u) | ((inr && inb) || q3 <= t2 ? 8u : 0u);
 }
 
+// The same test for one quadrant, pixel (px0, py0) its first.
+__device__ __forceinline__ bool quadrant_reached(float x, float y, float4 c, int px0, int py0) {
+    const float o = c.w;
+    if (!(o >= 0.0039215f)) return !(o == o);  // alpha < 1/255 everywhere
+    const float A = c.x, B = c.y, C = c.z;
+    const float det = fmaf(A, C, -B * B);
+    if (!(A > 0.0f && C > 0.0f && det > 1e-3f * A * C)) return true;
+    const float t2 = 2.0f * fmaf(ln_fast(255.0f * o), 1.01f, 1e-3f);
+    if (!(t2 < 1e30f && A < 1e30f && C < 1e30f && fabsf(x) < 1e30f && fabsf(y) < 1e30f))
+        return true;
+    const float ia = __builtin_amdgcn_rcpf(A), ic = __builtin_amdgcn_rcpf(C);
+    const float x0 = ((float)px0 + 0.5f) - x, x1 = x0 + 7.0f;
+    const float y0 = ((float)py0 + 0.5f) - y, y1 = y0 + 7.0f;
+    // the row and the column edge nearer the mean
+    const float ky = y1 < 0.0f ? y1 : y0, kx = x1 < 0.0f ? x1 : x0;
+    const float xs = -B * ia * ky, u = fminf(fmaxf(xs, x0), x1) - xs;
+    const float ys = -B * ic * kx, v = fminf(fmaxf(ys, y0), y1) - ys;
+    const float q = fminf(fmaf(A * u, u, ky * ky * (det * ia)), fmaf(C * v, v, kx * kx * (det * ic)));
+    return (x0 <= 0.0f && x1 >= 0.0f && y0 <= 0.0f && y1 >= 0.0f) || q <= t2;
+}
+
 // A staged Gaussian is "plain" when every quantity the per-pixel loop reads
 // is finite and small enough that the float32 power is finite and, for a
 // pixel that passes the alpha bound, within [-86, 0]: then exp needs no
@@ -226,37 +249,6 @@ __device__ __forceinline__ float dpp_f(float v) {
         }                                                                                    \
     } while (0)
 
-// The last two steps of a 16-lane row sum for K registers, up to four per
-// asm block: t[k] += t[k] of the mirrored lane of its 8-lane half-row (DPP
-// row_half_mirror), then += that of the mirrored lane of its row
-// (row_mirror), after which every lane of a row holds the row's total.
-// asm (volatile) so the adds are not sunk into the following one-lane store
-// branch, where each would become a DPP move with a zero fill plus a
-// separate add; s_nop 1 gives the two wait states a DPP read needs after a
-// VALU write of its operand.
-#define GSX_DPP_ADD(r, ctl) "v_add_f32_dpp " r ", " r ", " r " " ctl " row_mask:0xf bank_mask:0xf\n\t"
-#define GSX_ROW_TAIL1(ctl) GSX_DPP_ADD("%0", ctl)
-#define GSX_ROW_TAIL2(ctl) GSX_DPP_ADD("%0", ctl) GSX_DPP_ADD("%1", ctl)
-#define GSX_ROW_TAIL3(ctl) GSX_DPP_ADD("%0", ctl) GSX_DPP_ADD("%1", ctl) GSX_DPP_ADD("%2", ctl)
-#define GSX_ROW_TAIL4(ctl) \
-    GSX_DPP_ADD("%0", ctl) GSX_DPP_ADD("%1", ctl) GSX_DPP_ADD("%2", ctl) GSX_DPP_ADD("%3", ctl)
-#define GSX_ROW_TAIL(N)                                                                   \
-    "s_nop 1\n\t" GSX_ROW_TAIL##N("row_half_mirror") "s_nop 1\n\t" GSX_ROW_TAIL##N("row_mirror")
-
-template <int K>
-__device__ __forceinline__ void row_tail_add(float (&t)[K]) {
-    static_assert(K >= 1 && K <= 4, "one to four registers per block");
-    if constexpr (K == 4) {
-        asm volatile(GSX_ROW_TAIL(4) : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3]));
-    } else if constexpr (K == 3) {
-        asm volatile(GSX_ROW_TAIL(3) : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]));
-    } else if constexpr (K == 2) {
-        asm volatile(GSX_ROW_TAIL(2) : "+v"(t[0]), "+v"(t[1]));
-    } else {
-        asm volatile(GSX_ROW_TAIL(1) : "+v"(t[0]));
-    }
-}
-
 template <int K>
 __device__ __forceinline__ void swap_rows32(float (&a)[K], float (&b)[K]) {
     GSX_SWAP_BLOCK("v_permlane32_swap_b32", K, a, b);
@@ -266,15 +258,13 @@ __device__ __forceinline__ void swap_rows16(float (&a)[K], float (&b)[K]) {
     GSX_SWAP_BLOCK("v_permlane16_swap_b32", K, a, b);
 }
 
-// Sums of NVP per-lane values (NVP a multiple of 4) over the 64 lanes of
-// the wave, spread over the four 16-lane rows: afterwards every lane of row
-// r holds in q[m] the total of value 4m + row_value(r).  Step 1 swaps the
-// upper half of value 2k with the lower half of value 2k + 1 and adds, so
-// each half carries one of the two values; step 2 does the same between
-// rows; step 3 sums each row with four DPP steps.  NVP + NVP/2 + NVP
-// exchanges/adds instead of 6 NVP for a separate 64-lane reduction of every
-// value.  Values from index NZ on are known zeros: pairs of them skip their
-// exchange.  All lanes must be active.
+// Sums of NVP per-lane values (NVP a multiple of 4) over the four 16-lane
+// rows of the wave, spread over the rows: after the two steps every lane of
+// row r holds in q[m] its column's total of value 4m + row_value(r).  Step 1
+// swaps the upper half of value 2k with the lower half of value 2k + 1 and
+// adds, so each half carries one of the two values; step 2 does the same
+// between rows.  Values from index NZ on are known zeros: pairs of them skip
+// their exchange.  All lanes must be active.
 __device__ __forceinline__ int row_value(int row) { return ((row & 1) << 1) | (row >> 1); }
 
 // Step 1 for value pairs K0..K1-1: h[k] = swap32-sum of v[2k], v[2k + 1]
@@ -313,47 +303,6 @@ __device__ __forceinline__ void reduce_step2(const float (&h)[NVP / 2], float (&
         for (int k = 0; k < N; ++k) q[M0 + k] = a[k] + b[k];
         reduce_step2<M0 + N, M1, NVP>(h, q);
     }
-}
-
-// Steps 2 and 3 for row groups M0..M1-1: swap16-sum of h[2m], h[2m + 1],
-// then the four DPP steps within each row.
-template <int M0, int M1, int NVP>
-__device__ __forceinline__ void reduce_step23(const float (&h)[NVP / 2], float (&q)[NVP / 4]) {
-    if constexpr (M0 < M1) {
-        constexpr int N = (M1 - M0) < 4 ? (M1 - M0) : 4;
-        float a[N], b[N];
-#pragma unroll
-        for (int k = 0; k < N; ++k) {
-            a[k] = h[2 * (M0 + k)];
-            b[k] = h[2 * (M0 + k) + 1];
-        }
-        swap_rows16<N>(a, b);
-#pragma unroll
-        for (int k = 0; k < N; ++k) {
-            float t = a[k] + b[k];
-            t += dpp_f<0xB1, 0xF, 0xF>(t);  // quad_perm [1,0,3,2]
-            t += dpp_f<0x4E, 0xF, 0xF>(t);  // quad_perm [2,3,0,1]
-            a[k] = t;
-        }
-        row_tail_add<N>(a);
-#pragma unroll
-        for (int k = 0; k < N; ++k) q[M0 + k] = a[k];
-        reduce_step23<M0 + N, M1, NVP>(h, q);
-    }
-}
-
-template <int NVP, int NZ = NVP>
-__device__ __forceinline__ void wave_reduce_rows(const float (&v)[NVP], float (&q)[NVP / 4]) {
-    static_assert(NVP % 4 == 0 && NZ <= NVP, "values come in groups of four");
-    constexpr int K1 = (NZ + 1) / 2;  // value pairs with a non-zero member
-    constexpr int K2 = (K1 + 1) / 2;  // row groups with a non-zero member
-    float h[NVP / 2];
-#pragma unroll
-    for (int k = K1; k < NVP / 2; ++k) h[k] = 0.0f;
-    reduce_step1<0, K1, NVP, NZ>(v, h);
-#pragma unroll
-    for (int m = K2; m < NVP / 4; ++m) q[m] = 0.0f;
-    reduce_step23<0, K2, NVP>(h, q);
 }
 
 __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
@@ -802,26 +751,6 @@ __device__ __forceinline__ float* slot_at(float4 (*part)[((CH + 6) + 3) / 4], in
     return reinterpret_cast<float*>(reinterpret_cast<char*>(part) + off * NV4);
 }
 
-// Wave sums of one Gaussian's values into its slot: row r of the wave ends
-// with the totals of values 4m + row_value(r), which lane 15 of the row
-// stores at those positions.
-template <int CH>
-__device__ __forceinline__ void bwd_reduce1(const float (&v)[CH + 6], int off,
-                                            float4 (*part)[((CH + 6) + 3) / 4], int lane) {
-    constexpr int NV = CH + 6;
-    constexpr int NVP = 4 * ((NV + 3) / 4);
-    float w[NVP];
-#pragma unroll
-    for (int q = 0; q < NVP; ++q) w[q] = q < NV ? v[q] : 0.0f;
-    float tot[NVP / 4];
-    wave_reduce_rows<NVP, NV>(w, tot);
-    if ((lane & 15) == 15) {
-        float* dst = slot_at<CH>(part, off) + row_value(lane >> 4);
-#pragma unroll
-        for (int m = 0; m < NVP / 4; ++m) dst[4 * m] = tot[m];
-    }
-}
-
 // The same for two different Gaussians in one reduction (fewer padding
 // values and shared exchange steps): value i of Gaussian a sits at 2i and of
 // Gaussian b at 2i + 1 of the combined array, so the first exchange pairs
@@ -840,7 +769,7 @@ __device__ __forceinline__ void bwd_reduce2(float (&w)[4 * ((CH + 7) / 2)], int 
 #pragma unroll
     for (int k = K1; k < 2 * NH; ++k) h[k] = 0.0f;
     reduce_step1<0, K1, 4 * NH, 2 * NV>(w, h);
-    // step 2 (swap16-sum between rows) as in wave_reduce_rows: a[m] holds in
+    // step 2 (swap16-sum between rows): a[m] holds in
     // row r the row's partial of value 4m + row_value(r)
     float a[NH];
 #pragma unroll
@@ -911,43 +840,6 @@ __device__ __forceinline__ void bwd_reduce2(float (&w)[4 * ((CH + 7) / 2)], int 
     }
 }
 
-// Back-to-front walk of one quadrant wave over its list (descending staged
-// index), records and list entries read ahead as in fwd_walk, one
-// reduction per contributing Gaussian.
-template <int CH, bool PLAIN>
-__device__ __forceinline__ void bwd_walk1(const uint32_t* list, int cnt, int lim,
-                                          const float4* s_r0, const float4* s_r1,
-                                          const float4 (*s_f)[(CH + 3) / 4],
-                                          float4 (*part)[((CH + 6) + 3) / 4], float pxf,
-                                          float pyf, int lane, BwdPixel<CH>& px) {
-    constexpr int F4 = (CH + 3) / 4;
-    const float4* sf = &s_f[0][0];
-    if (cnt <= 0) return;
-    int oa = list[0], ob = list[1];
-    float4 a0 = rec_at(s_r0, oa), a1 = rec_at(s_r1, oa);
-    for (int i = 0;; i += 2) {
-        const int na = list[i + 2];
-        const float4 b0 = rec_at(s_r0, ob), b1 = rec_at(s_r1, ob);
-        {
-            float v[CH + 6];
-            if (bwd_values<CH, PLAIN>(a0, a1, &rec_at(sf, oa * F4), oa, lim, pxf, pyf, px, v))
-                bwd_reduce1<CH>(v, oa, part, lane);
-        }
-        if (i + 1 >= cnt) return;
-        const int nb = list[i + 3];
-        a0 = rec_at(s_r0, na);
-        a1 = rec_at(s_r1, na);
-        {
-            float v[CH + 6];
-            if (bwd_values<CH, PLAIN>(b0, b1, &rec_at(sf, ob * F4), ob, lim, pxf, pyf, px, v))
-                bwd_reduce1<CH>(v, ob, part, lane);
-        }
-        if (i + 2 >= cnt) return;
-        oa = na;
-        ob = nb;
-    }
-}
-
 // The same walk two Gaussians at a time, the pair sharing one reduction (a
 // Gaussian without contributions enters it as zeros): their values are
 // written interleaved, a's at even and b's at odd positions, which is the
@@ -955,7 +847,7 @@ __device__ __forceinline__ void bwd_walk1(const uint32_t* list, int cnt, int lim
 // the next a's before b is.  An odd count pairs the last Gaussian with the
 // padding record, which contributes nothing and owns a slot of its own.
 template <int CH, bool PLAIN>
-__device__ __forceinline__ void bwd_walk2(const uint32_t* list, int cnt, int lim,
+__device__ __forceinline__ void bwd_walk(const uint32_t* list, int cnt, int lim,
                                           const float4* s_r0, const float4* s_r1,
                                           const float4 (*s_f)[(CH + 3) / 4],
                                           float4 (*part)[((CH + 6) + 3) / 4], float pxf,
@@ -984,29 +876,12 @@ __device__ __forceinline__ void bwd_walk2(const uint32_t* list, int cnt, int lim
     }
 }
 
-// Paired reductions up to four channels (at most 20 values per pair); wider
-// channel blocks reduce one Gaussian at a time, where padding is a small
-// share and two value sets would not fit the register budget.
-template <int CH, bool PLAIN>
-__device__ __forceinline__ void bwd_walk(const uint32_t* list, int cnt, int lim,
-                                         const float4* s_r0, const float4* s_r1,
-                                         const float4 (*s_f)[(CH + 3) / 4],
-                                         float4 (*part)[((CH + 6) + 3) / 4], float pxf, float pyf,
-                                         int lane, BwdPixel<CH>& px) {
-    if constexpr (CH <= 4)
-        bwd_walk2<CH, PLAIN>(list, cnt, lim, s_r0, s_r1, s_f, part, pxf, pyf, lane, px);
-    else
-        bwd_walk1<CH, PLAIN>(list, cnt, lim, s_r0, s_r1, s_f, part, pxf, pyf, lane, px);
-}
-
 // Waves per SIMD the backward asks for (more waves hide LDS and ballot
 // latencies): six at one and three channels (<= 80 VGPRs, 12-16 KB of LDS),
-// five at two and four channels (which would spill at 80), four up to 16
-// channels, three at 32; no instantiation spills (checked with
-// -Rpass-analysis=kernel-resource-usage: ScratchSize 0 for every one).
-constexpr int bwd_min_waves(int ch) {
-    return (ch == 2 || ch == 4) ? 5 : (ch <= 4 ? 6 : (ch <= 16 ? 4 : 3));
-}
+// five at two and four channels (which would spill at 80); no instantiation
+// spills (checked with -Rpass-analysis=kernel-resource-usage: ScratchSize 0
+// for every one).
+constexpr int bwd_min_waves(int ch) { return (ch == 2 || ch == 4) ? 5 : 6; }
 
 template <int CH>
 __global__ __launch_bounds__(kThreads, bwd_min_waves(CH)) void k_raster_bwd(
@@ -1205,472 +1080,687 @@ __global__ __launch_bounds__(kThreads, bwd_min_waves(CH)) void k_raster_bwd(
             const int g = __float_as_int(s_r1[j].w);
             const float v = reinterpret_cast<const float*>(s_part[0][j])[k];
             if (g < 0 || v == 0.0f || (k >= 6 && k - 6 >= nc)) continue;
-            float* dst = gstride > 0 ? g_xy + (int64_t)gstride * g + (k < 6 ? k : c0 + k)
-                       : k < 2 ? g_xy + 2 * (int64_t)g + k
-                       : k < 5 ? g_conic + 3 * (int64_t)g + (k - 2)
-                       : k == 5 ? g_opac + g
-                                : g_feat + (int64_t)g * C + c0 + (k - 6);
-            atomicAdd(dst, v);
-        }
-    }
-}
-
-// ------------------------------------------------- matrix-core backward --
-// The backward for wide channel blocks (CH = 32) with its channel work on
-// the matrix cores.  Per (Gaussian, pixel) pair the replay is the same VALU
-// arithmetic as bwd_values -- every alpha / T / early-stop decision and the
-// per-pixel running state are unchanged -- except that the two channel
-// contractions come from v_mfma_f32_16x16x4_f32 products over groups of 16
-// list entries:
-//   A. cg[g][p] = sum_c f[g][c] g[p][c], (16 x 32) x (32 x 64), before the
-//      group's replay (the features are staged; the pixels' cotangents are
-//      held in registers in the B-operand layout for the whole walk), and
-//   B. dL/dc[g][c] = sum over the wave's 64 pixels of aT[g][p] g[p][c],
-//      (16 x 64) x (64 x 32), after it (aT = alpha T of each pair).
-// One LDS tile per wave carries cg[g][p] to the replay, which overwrites
-// entry (g, p) with aT[g][p] once read.  The replay itself produces only
-// the six geometric values (u, w, u dx, u dy, w dy, G dL/dalpha), reduced
-// across the wave as before.  Operand layouts (checked on the GPU):
-// A[row = l % 16][k = l / 16], B[k = l / 16][col = l % 16]; the result's lane
-// l holds rows 4 (l / 16) + i, column l % 16.  The features are staged
-// channel-major (row stride 65) and the tile with row stride 68, so the
-// operand reads and result writes of a wave hit distinct LDS banks.  The
-// geometric sums of the four quadrant waves meet in one LDS slot per
-// Gaussian through LDS float atomics (three per pair); product B's channel
-// sums go straight to the gradient record with global float atomics, one
-// instruction covering four Gaussians' 16 consecutive channels -- LDS
-// float atomics for them (eight per group and lane) cost more than the
-// whole global flush, and per-wave LDS slots instead (34 KB) cut the
-// workgroups per CU from three to two, slower still.  The contractions add
-// in a different order than the VALU path, so gradients agree with it to
-// float32 rounding, not bitwise; no decision depends on them.
-constexpr int kMxGroup = 16;   // Gaussians per matrix-core group
-constexpr int kMxPad = 68;     // row stride (floats) of a wave's tile: 4 r + q bank spread
-constexpr int kMxFPad = 65;    // row stride (floats) of the channel-major features
-constexpr int kMxGeo = 6;      // geometric values per Gaussian
-constexpr int kMxGeoStride = 8;   // slot stride (floats) of the geometric sums
-
-// Where a Gaussian's feature gradients go: base + stride * id + offset + c
-// for channels c < nc of the block.
-struct MxFeatOut {
-    float* base;
-    int64_t stride;
-    int offset;
-    int nc;
-};
-
-typedef float mx_floatx4 __attribute__((ext_vector_type(4)));
-
-struct MxPixel {
-    float T;  // transmittance in front of the current Gaussian
-    float Q;
-    int last;
-};
-
-// The replay of one (pixel, Gaussian) pair given cg = c . g: the geometric
-// values into v (zeros where the pixel does not composite the Gaussian) and
-// alpha T into aT (zero likewise).  Returns whether any lane of the wave
-// passes the first tests (v and aT are zero when it does not).
-template <bool PLAIN>
-__device__ __forceinline__ bool bwd_geo(const float4& r0, const float4& r1, float cg, int off,
-                                        int lim, float pxf, float pyf, MxPixel& px,
-                                        float (&v)[8], float& aT_out) {
-    const float dx = r0.x - pxf, dy = r0.y - pyf;
-    const float power = splat_power(r1.x, r1.y, r1.z, dx, dy);
-    // PLAIN: the power is never positive (plain_gaussian's conic bound)
-    const bool c1 = off < lim, c2 = PLAIN || !(power > 0.0f), c3 = !(power < r0.z);
-    bool ok = c1 && c2 && c3;
-    const uint64_t m123 = PLAIN ? __ballot(c1) & __ballot(c3)
-                                : __ballot(c1) & __ballot(c2) & __ballot(c3);
-#pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = 0.0f;
-    aT_out = 0.0f;
-    if (m123 == 0ull) return false;
-    const float G = PLAIN ? splat_exp_core(power) : splat_exp_sel(power);
-    const float alpha = fminf(0.99f, r0.w * G);
-    const bool c4 = !(alpha < 1.0f / 255.0f);
-    ok = ok && c4;
-    if ((m123 & __ballot(c4)) == 0ull) return false;
-    float ga, aT;
-    if constexpr (PLAIN) {
-        const float Gs = ok ? G : 0.0f;
-        const float as = ok ? alpha : 0.0f;
-        const float rcp = __builtin_amdgcn_rcpf(1.0f - as);
-        px.T = px.T * rcp;
-        const float dL_dalpha = fmaf(cg, px.T, -(px.Q * rcp));
-        aT = as * px.T;
-        px.Q = fmaf(aT, cg, px.Q);
-        ga = Gs * dL_dalpha;
-    } else {
-        const float rcp = __builtin_amdgcn_rcpf(1.0f - alpha);
-        px.T = ok ? px.T * rcp : px.T;
-        float dL_dalpha = fmaf(cg, px.T, -(px.Q * rcp));
-        dL_dalpha = ok ? dL_dalpha : 0.0f;
-        aT = ok ? alpha * px.T : 0.0f;
-        px.Q = ok ? fmaf(aT, cg, px.Q) : px.Q;
-        ga = G * dL_dalpha;
-    }
-    const float u = ga * dx, w = ga * dy;
-    v[0] = (PLAIN || ok) ? u : 0.0f;
-    v[1] = (PLAIN || ok) ? w : 0.0f;
-    v[2] = (PLAIN || ok) ? u * dx : 0.0f;
-    v[3] = (PLAIN || ok) ? u * dy : 0.0f;
-    v[4] = (PLAIN || ok) ? w * dy : 0.0f;
-    v[5] = (PLAIN || ok) ? ga : 0.0f;
-    aT_out = aT;  // zero for lanes that do not composite (PLAIN: as = 0)
-    return true;
-}
-
-// The walk of one quadrant wave for the matrix-core backward: groups of up
-// to 16 list entries (back to front): product A into the tile, the replay
-// pair by pair, product B into the Gaussians' LDS slots.  gA[pb][ks] =
-// g(pixel 16 pb + l % 16, channel 4 ks + l / 16); gB[ks][cb] = g(pixel
-// 4 ks + l / 16, channel 16 cb + l % 16).
-template <bool PLAIN>
-__device__ __forceinline__ void bwd_walk_mx(const uint32_t* list, int cnt, int lim,
-                                            const float4* s_r0, const float4* s_r1,
-                                            const float* s_feat, int pad_slot,
-                                            float (*sum)[kMxGeoStride], const MxFeatOut& fo,
-                                            float (*tile)[kMxPad],
-                                            const float (&gA)[4][8], const float (&gB)[16][2],
-                                            float pxf, float pyf, int lane, MxPixel& px) {
-#pragma unroll 1
-    for (int i0 = 0; i0 < cnt; i0 += kMxGroup) {
-        const int ng = min(kMxGroup, cnt - i0);
-        // A: the features of entry l % 16 (the padding record's zeros past
-        // the group), channels 4 ks + l / 16
-        const int row = lane & 15;
-        const int slot = row < ng ? (list[i0 + row] >> 4) : pad_slot;
-        float fa[8];
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) fa[ks] = s_feat[(4 * ks + (lane >> 4)) * kMxFPad + slot];
-#pragma unroll
-        for (int pb = 0; pb < 4; ++pb) {
-            mx_floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int ks = 0; ks < 8; ++ks)
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[ks], gA[pb][ks], acc, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) tile[4 * (lane >> 4) + i][16 * pb + row] = acc[i];
-        }
-        // the wave's LDS accesses complete in order; the fence keeps the
-        // compiler from moving the reads below above the writes
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        // the replay two entries at a time (a = j, b = j + 1; past the group
-        // the padding record, which contributes nothing), their geometric
-        // values interleaved (a's at even, b's at odd positions) into one
-        // reduction, the next pair's records read before this pair is
-        // evaluated
-        const int pad = pad_slot * 16;
-        int oa = 0 < ng ? list[i0] : pad, ob = 1 < ng ? list[i0 + 1] : pad;
-        float4 a0 = rec_at(s_r0, oa), a1 = rec_at(s_r1, oa);
-        float4 b0 = rec_at(s_r0, ob), b1 = rec_at(s_r1, ob);
-        float cga = tile[0][lane], cgb = tile[1][lane];
-#pragma unroll 1
-        for (int j = 0; j < kMxGroup; j += 2) {
-            const int na = j + 2 < ng ? list[i0 + j + 2] : pad;
-            const int nb = j + 3 < ng ? list[i0 + j + 3] : pad;
-            // the next pair's rows are not overwritten before they are read
-            const float nca = j + 2 < kMxGroup ? tile[j + 2][lane] : 0.0f;
-            const float ncb = j + 3 < kMxGroup ? tile[j + 3][lane] : 0.0f;
-            float va[8], vb[8], aTa, aTb;
-            const bool ha = bwd_geo<PLAIN>(a0, a1, cga, oa, lim, pxf, pyf, px, va, aTa);
-            const bool hb = bwd_geo<PLAIN>(b0, b1, cgb, ob, lim, pxf, pyf, px, vb, aTb);
-            tile[j][lane] = aTa;
-            tile[j + 1][lane] = aTb;
-            a0 = rec_at(s_r0, na);
-            a1 = rec_at(s_r1, na);
-            b0 = rec_at(s_r0, nb);
-            b1 = rec_at(s_r1, nb);
-            if (ha || hb) {
-                float w[12], h[6], q[3];
-#pragma unroll
-                for (int k = 0; k < kMxGeo; ++k) {
-                    w[2 * k] = va[k];
-                    w[2 * k + 1] = vb[k];
-                }
-                reduce_step1<0, 6, 12, 12>(w, h);
-                reduce_step2<0, 3, 12>(h, q);
-                // within the row: q[0], q[1] exchanged by halving over
-                // row_mirror (lanes 8..15 keep q[1]), q[2] summed whole;
-                // rows with row_value 0 and 2 hold a's values 2m and 2m + 1,
-                // rows with 1 and 3 b's
-                const bool hi8 = (lane & 8) != 0;
-                const float x = hi8 ? q[1] : q[0], y = hi8 ? q[0] : q[1];
-                float b = x + dpp_f<0x140, 0xF, 0xF>(y);  // row_mirror
-                float c = q[2] + dpp_f<0x140, 0xF, 0xF>(q[2]);
-                b += dpp_f<0x141, 0xF, 0xF>(b);  // row_half_mirror
-                c += dpp_f<0x141, 0xF, 0xF>(c);
-                b += dpp_f<0xB1, 0xF, 0xF>(b);  // quad_perm [1,0,3,2]
-                c += dpp_f<0xB1, 0xF, 0xF>(c);
-                b += dpp_f<0x4E, 0xF, 0xF>(b);  // quad_perm [2,3,0,1]
-                c += dpp_f<0x4E, 0xF, 0xF>(c);
-                asm volatile("" ::"v"(b), "v"(c));
-                const int rv = row_value(lane >> 4);
-                float* dst = sum[((rv & 1) ? ob : oa) >> 4] + (rv >> 1);
-                if ((lane & 7) == 7) atomicAdd(dst + (hi8 ? 2 : 0), b);
-                if ((lane & 15) == 15) atomicAdd(dst + 4, c);
-            }
-            oa = na;
-            ob = nb;
-            cga = nca;
-            cgb = ncb;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        mx_floatx4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int ks = 0; ks < 16; ++ks) {
-            const float a = tile[row][4 * ks + (lane >> 4)];
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a, gB[ks][0], acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a, gB[ks][1], acc1, 0, 0, 0);
-        }
-        // lane l holds the sums of entries 4 (l / 16) + i, channels l % 16
-        // and 16 + l % 16: added straight into the Gaussians' feature
-        // gradients (one instruction covers four Gaussians' 16 consecutive
-        // channels; zero sums are skipped)
-        const uint4 gl = *reinterpret_cast<const uint4*>(list + i0 + 4 * (lane >> 4));
-        const uint32_t gi[4] = {gl.x, gl.y, gl.z, gl.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int g = 4 * (lane >> 4) + i;
-            if (g < ng) {
-                const int gid = __float_as_int(s_r1[gi[i] >> 4].w);
-                float* dst = fo.base + (int64_t)fo.stride * gid + fo.offset + row;
-                if (acc0[i] != 0.0f && row < fo.nc) atomicAdd(dst, acc0[i]);
-                if (acc1[i] != 0.0f && row + 16 < fo.nc) atomicAdd(dst + 16, acc1[i]);
-            }
-        }
-        // the next group's product A overwrites the tile
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    }
-}
-
-template <int CH>
-__global__ __launch_bounds__(kThreads, 3) void k_raster_bwd_mx(
-    const float2* __restrict__ xy, const float4* __restrict__ co, const float* __restrict__ feat,
-    int C, int c0, int nc, const int* __restrict__ ids, const int2* __restrict__ ranges,
-    int64_t n, int64_t n_ids, const float* __restrict__ bg, int W, int H, int tiles_x,
-    const float* __restrict__ final_T, const int* __restrict__ n_contrib,
-    const float* __restrict__ grad_out, const float* __restrict__ grad_T,
-    float* __restrict__ g_xy, float* __restrict__ g_conic, float* __restrict__ g_feat,
-    float* __restrict__ g_opac, int gstride, const int* __restrict__ order) {
-    static_assert(CH == 32, "the matrix-core backward covers 32-channel blocks");
-    constexpr int F4 = CH / 4;
-    constexpr int BB = 64;
-    constexpr int NLW = BB / kWave;
-    __shared__ float4 s_r0[BB + 1];
-    __shared__ float4 s_r1[BB + 1];  // -a/2, -b, -c/2 (conic), Gaussian id (int bits)
-    __shared__ float s_fT[CH * kMxFPad];              // features, channel-major (column BB: zeros)
-    __shared__ float s_sum[BB + 1][kMxGeoStride];     // geometric sums over the waves
-    __shared__ float s_tile[kWaves][kMxGroup][kMxPad];  // per-wave cg / aT tiles
-    __shared__ uint64_t s_mask[kWaves][NLW];
-    // walk lists; a group's 16 entries are read as four 16-byte pieces, so
-    // each row has room for a whole group past the last entry
-    __shared__ __align__(16) uint32_t s_list[kWaves][BB + kMxGroup];
-    __shared__ int s_last[kWaves];
-    __shared__ __align__(16) uint32_t s_plain[kWaves];
-
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int tile = __builtin_amdgcn_readfirstlane(tile_at(order, blockIdx.x, gridDim.x, true));
-    if (tile < 0) return;  // past the end of this XCD's band
-    // rows of CH channels at 16-byte aligned addresses: float4 loads
-    const bool vec4 = nc >= CH && ((C | c0) & 3) == 0 && ((uintptr_t)feat & 15u) == 0;
-    const int tx = tile % tiles_x, ty = tile / tiles_x;
-    const int px0 = tx * kTile, py0 = ty * kTile;
-    const int qx0 = px0 + (wave & 1) * 8, qy0 = py0 + (wave >> 1) * 8;
-    const int px = qx0 + (lane & 7);
-    const int py = qy0 + (lane >> 3);
-    const bool inside = px < W && py < H;
-    const float pxf = (float)px + 0.5f, pyf = (float)py + 0.5f;
-    const int64_t pid = (int64_t)py * W + px;
-
-    int start, num;
-    tile_span(ranges[tile], n_ids, start, num);
-
-    MxPixel st;
-    // the pixel's loads issue together (clamped indices, masked after)
-    const int64_t pidc = inside ? pid : 0;
-    const float tf = final_T[pidc];
-    const int nct = n_contrib[pidc];
-    const float gt = grad_T ? grad_T[pidc] : 0.0f;
-    const float T_final = inside ? tf : 1.0f;
-    st.T = T_final;
-    st.last = inside ? nct : 0;
-    float bg_dot = 0.0f;
-    {
-        float gp[CH], bgv[CH];
-#pragma unroll
-        for (int ch = 0; ch < CH; ++ch) {
-            gp[ch] = grad_out[pidc * C + c0 + min(ch, nc - 1)];
-            bgv[ch] = bg ? bg[c0 + min(ch, nc - 1)] : 0.0f;
-        }
-#pragma unroll
-        for (int ch = 0; ch < CH; ++ch)
-            if (ch < nc) bg_dot = bg_dot + bgv[ch] * (inside ? gp[ch] : 0.0f);
-    }
-    if (inside && c0 == 0 && grad_T) bg_dot = bg_dot + gt;
-    st.Q = T_final * bg_dot;
-    // the quadrant's cotangents in the two B-operand layouts (pixel q of
-    // the quadrant is (q % 8, q / 8))
-    auto gval = [&](int q, int ch) {
-        const int bx = qx0 + (q & 7), by = qy0 + (q >> 3);
-        return (bx < W && by < H && ch < nc) ? grad_out[((int64_t)by * W + bx) * C + c0 + ch]
-                                             : 0.0f;
-    };
-    float gA[4][8], gB[16][2];
-#pragma unroll
-    for (int pb = 0; pb < 4; ++pb)
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) gA[pb][ks] = gval(16 * pb + (lane & 15), 4 * ks + (lane >> 4));
-#pragma unroll
-    for (int ks = 0; ks < 16; ++ks)
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) gB[ks][cb] = gval(4 * ks + (lane >> 4), 16 * cb + (lane & 15));
-
-    if (tid == 0) {
-        s_r0[BB] = make_float4(0.0f, 0.0f, __builtin_huge_valf(), 0.0f);
-        s_r1[BB] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-    if (tid < CH) s_fT[tid * kMxFPad + BB] = 0.0f;
-    {
-        int m = st.last;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, kWave));
-        if (lane == 0) s_last[wave] = m;
-    }
-    __syncthreads();
-    int quad_last[kWaves];
-#pragma unroll
-    for (int q = 0; q < kWaves; ++q) quad_last[q] = s_last[q];
-    const int max_last = max(max(quad_last[0], quad_last[1]), max(quad_last[2], quad_last[3]));
-    const int n_batches = (max_last + BB - 1) / BB;
-    const MxFeatOut fout = gstride > 0 ? MxFeatOut{g_xy, gstride, kMxGeo + c0, nc}
-                                       : MxFeatOut{g_feat, C, c0, nc};
-
-    for (int b = n_batches - 1; b >= 0; --b) {
-        __syncthreads();
-        uint32_t qm = 0;
-        bool plain = true;
-        for (int k = tid; k < (BB + 1) * kMxGeoStride; k += kThreads) (&s_sum[0][0])[k] = 0.0f;
-        if (tid < BB) {
-            const int k = b * BB + tid;
-            float4 r1 = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(-1));
-            if (k < num) {
-                const int g = ids[start + k];
-                if ((uint32_t)g < (uint64_t)n) {
-                    const float2 m = xy[g];
-                    const float4 c = co[g];
-                    const float thr = alpha_floor_power(c.w);
-                    s_r0[tid] = make_float4(m.x, m.y, thr, c.w);
-                    r1 = make_float4(-0.5f * c.x, -c.y, -0.5f * c.z, __int_as_float(g));
-                    qm = quadrant_mask(m.x, m.y, c, px0, py0);
-#pragma unroll
-                    for (int q = 0; q < kWaves; ++q)
-                        if (k >= quad_last[q]) qm &= ~(1u << q);
-                    plain = plain_gaussian<0>(m.x, m.y, c, thr, nullptr);
-                }
-            }
-            s_r1[tid] = r1;
-        }
-        if (wave < NLW) {
-#pragma unroll
-            for (int q = 0; q < kWaves; ++q) {
-                const uint64_t bq = __ballot((qm >> q) & 1u);
-                if (lane == 0) s_mask[q][wave] = bq;
-            }
-        }
-        // the features: every thread stages two of the batch's float4
-        // pieces (the ids come from the records above), so no thread holds a
-        // Gaussian's 32 channels beside the walk's cotangent registers
-        __syncthreads();
-        if (vec4) {
-            // whole aligned rows: the 16-byte loads issue together (entries
-            // without a Gaussian read row 0 and are dropped)
-            constexpr int NIT = BB * F4 / kThreads;
-            static_assert(BB * F4 % kThreads == 0, "whole rounds");
-            int g[NIT];
-            float4 v[NIT];
-#pragma unroll
-            for (int it = 0; it < NIT; ++it) {
-                const int k = tid + it * kThreads, j = k / F4, q = k - j * F4;
-                g[it] = __float_as_int(s_r1[j].w);
-                const int64_t gi = g[it] >= 0 ? g[it] : 0;
-                v[it] = *reinterpret_cast<const float4*>(feat + gi * C + c0 + 4 * q);
-            }
-#pragma unroll
-            for (int it = 0; it < NIT; ++it) {
-                const int k = tid + it * kThreads, j = k / F4, q = k - j * F4;
-                if (g[it] >= 0) {
-                    float* d = s_fT + (4 * q) * kMxFPad + j;
-                    d[0] = v[it].x;
-                    d[kMxFPad] = v[it].y;
-                    d[2 * kMxFPad] = v[it].z;
-                    d[3 * kMxFPad] = v[it].w;
-                    plain = plain && fabsf(v[it].x) < 1e30f && fabsf(v[it].y) < 1e30f &&
-                            fabsf(v[it].z) < 1e30f && fabsf(v[it].w) < 1e30f;
-                }
-            }
-        } else
-        for (int k = tid; k < BB * F4; k += kThreads) {
-            const int j = k / F4, q = k - j * F4;
-            const int g = __float_as_int(s_r1[j].w);
-            if (g >= 0) {
-                const float* f = feat + (int64_t)g * C + c0 + 4 * q;
-                float4 v;
-                v.x = 4 * q < nc ? f[0] : 0.0f;
-                v.y = 4 * q + 1 < nc ? f[1] : 0.0f;
-                v.z = 4 * q + 2 < nc ? f[2] : 0.0f;
-                v.w = 4 * q + 3 < nc ? f[3] : 0.0f;
-                float* d = s_fT + (4 * q) * kMxFPad + j;
-                d[0] = v.x;
-                d[kMxFPad] = v.y;
-                d[2 * kMxFPad] = v.z;
-                d[3 * kMxFPad] = v.w;
-                plain = plain && fabsf(v.x) < 1e30f && fabsf(v.y) < 1e30f &&
-                        fabsf(v.z) < 1e30f && fabsf(v.w) < 1e30f;
-            }
-        }
-        const uint64_t np = __ballot(!plain);
-        if (lane == 0) s_plain[wave] = np == 0ull;
-        __syncthreads();
-        const uint4 pl = *reinterpret_cast<const uint4*>(s_plain);
-        const bool batch_plain = (pl.x & pl.y & pl.z & pl.w) != 0u;
-        const int cnt = build_list<NLW, true>(s_mask[wave], s_list[wave], lane, BB * 16);
-        const int lim = 16 * max(0, min(st.last - b * BB, BB));
-        const float* sfeat = s_fT;
-        if (batch_plain)
-            bwd_walk_mx<true>(s_list[wave], cnt, lim, s_r0, s_r1, sfeat, BB, s_sum, fout,
-                              s_tile[wave], gA, gB, pxf, pyf, lane, st);
-        else
-            bwd_walk_mx<false>(s_list[wave], cnt, lim, s_r0, s_r1, sfeat, BB, s_sum, fout,
-                               s_tile[wave], gA, gB, pxf, pyf, lane, st);
-        __syncthreads();
-        // one thread per Gaussian turns the sums into the reference's
-        // gradient components (rasterize.py:197-218 in terms of the sums)
-        if (tid < BB) {
-            float* e = s_sum[tid];
-            const float4 c = s_r1[tid];
-            const float o = s_r0[tid].w;
-            const float e0 = e[0], e1 = e[1];
-            e[0] = o * (2.0f * c.x * e0 + c.y * e1);
-            e[1] = o * (c.y * e0 + 2.0f * c.z * e1);
-            e[2] = -0.5f * o * e[2];
-            e[3] = -o * e[3];
-            e[4] = -0.5f * o * e[4];
-        }
-        __syncthreads();
-        for (int item = tid; item < BB * kMxGeo; item += kThreads) {
-            const int j = item / kMxGeo, k = item - j * kMxGeo;
-            const int g = __float_as_int(s_r1[j].w);
-            const float v = s_sum[j][k];
-            if (g < 0 || v == 0.0f) continue;
-            float* dst = gstride > 0 ? g_xy + (int64_t)gstride * g + k
+            float* dst = k >= 6 && g_feat ? g_feat + (int64_t)g * C + c0 + (k - 6)
+                       : gstride > 0 ? g_xy + (int64_t)gstride * g + (k < 6 ? k : c0 + k)
                        : k < 2 ? g_xy + 2 * (int64_t)g + k
                        : k < 5 ? g_conic + 3 * (int64_t)g + (k - 2)
                                 : g_opac + g;
             atomicAdd(dst, v);
         }
     }
+}
+
+typedef float mx_floatx4 __attribute__((ext_vector_type(4)));
+constexpr int kMxGroup = 16;   // Gaussians per matrix-core group
+
+// --------------------------------------- backward, five channels and more --
+// The same replay (a pixel's state is T and Q, BwdPixel) with the Gaussians
+// across the lanes.
+//
+// A quadrant wave takes its list 16 entries at a time (a bucket), lane l
+// holding entry l % 16 (0 the backmost), and steps over its 64 pixels four
+// at a time, row r = l / 16 of the wave working on one pixel: step s, row r
+// is pixel (s & 7, 4 (s >> 3) + r) of the quadrant.  Within a row, T in front
+// of each entry is the pixel's T times the inclusive product of the entries'
+// 1 / (1 - alpha), and Q behind it the pixel's Q plus the exclusive sum of
+// alpha T (c . g): two four-step DPP scans.  The Gaussian's gradient terms
+// then stay in its lane's registers over all the pixels, where lanes = pixels
+// has to sum every term of every Gaussian over the wave.  A column of steps is
+// skipped once its eight pixels have stopped in front of the bucket.
+//
+// Bound: the dependent instructions of a step (41 per 64 pairs; multiply-adds
+// take 2.4 cycles, DPP, compares, selects and minima 4.2 and the reciprocal
+// 8.3, measured) with 12 to 20 waves on a compute unit.  Measured against the
+// kernels before it (pixels across the lanes with the sums on the VALU up to
+// 16 channels; the channel products through an LDS tile, geometric sums
+// through LDS atomics, at 32): 500k Gaussians, 32 channels, 720p 509 -> 285
+// us; 60k, 12 channels, 641 x 479 182 -> 111 us; 200k surfels, 5 channels,
+// 960 x 540 224 -> 147 us (all with the geometric gradients in one record,
+// below).  With three channels it gains 5 % where Gaussians are small and
+// loses 18 % where they cover many tiles (every quadrant stages the list for
+// itself), so k_raster_bwd stays there.
+//
+// Along a column of the quadrant (steps x and x + 8) dx is shared, and a lane
+// only ever meets two rows, so the geometric terms are kept as moments in dx
+// per row, sum of h, h dx and h dx^2 (h = G dL/dalpha), and combined with the
+// rows' dy once per bucket.
+//
+// The channel work runs on the matrix cores (v_mfma_f32_16x16x4_f32, operand
+// A[row = l % 16][k = l / 16], B[k = l / 16][col = l % 16], result rows
+// 4 (l / 16) + i, column l % 16, checked on the GPU), whose layouts are the
+// replay's own, so nothing moves between lanes:
+//   c . g   A = g (16 pixels x 4 channels), B = c (4 channels x 16 entries):
+//           lane l gets its entry's product for the pixel of step i, row l / 16;
+//   dL/dc   A = g (16 channels x 4 pixels), B = alpha T of a step (4 pixels x
+//           16 entries, the lane's own value), accumulated over the steps.
+// No decision depends on them.
+constexpr int kBucket = 16;  // list entries per bucket (the lanes of a row)
+
+// Channel blocks of 5 to 8, 9 to 16 and 17 to 32 channels.
+template <int CHP>
+struct BwdShape {
+    static constexpr int BUF = 80;               // buffered entries: 15 left over + 64 new
+    static constexpr int KS = CHP / 4;           // k-steps of c . g
+    static constexpr int CB = (CHP + 15) / 16;   // 16-channel blocks of dL/dc
+    // up to 8 channels the cotangent operands are read from LDS where they
+    // are used (20 registers saved; dL/dc's rows past the channels hold
+    // copies, which nobody reads), wider blocks keep them in registers
+    static constexpr bool kNarrow = CHP <= 8;
+    static constexpr int NO = CHP + 8;  // row stride of a bucket's gradients in LDS
+};
+
+template <int V>
+using Int = std::integral_constant<int, V>;
+
+// The gradient outputs: the geometric ones in one record per Gaussian (xy,
+// stride floats) or in three arrays; feat + feat_stride * id + c is channel c
+// of the block, in the record or in an array of its own.
+struct BwdOut {
+    float* xy;
+    float* conic;
+    float* opac;
+    float* feat;
+    int64_t feat_stride;
+    int stride, nc, C;
+    bool record;   // geometric gradients in a record
+    bool whole;    // features in it too: sent together
+    int per, mul;  // entries per atomic instruction (64 / components), 65536 / components + 1
+};
+
+// Inclusive scans over the 16 lanes of each row, for two registers at once:
+// v <- v * (v of the lane 1, 2, 4, 8 below), sums likewise; lanes without a
+// partner keep their value.  A DPP read needs two wait states after the VALU
+// write of its operand, which the other register's step and an s_nop fill.
+#define GSX_SCAN_STEP(op, n)                                           \
+    op " %0, %0, %0 row_shr:" n " row_mask:0xf bank_mask:0xf\n\t"      \
+    op " %1, %1, %1 row_shr:" n " row_mask:0xf bank_mask:0xf\n\t"      \
+    "s_nop 0\n\t"
+#define GSX_SCAN(op)                                                   \
+    "s_nop 1\n\t" GSX_SCAN_STEP(op, "1") GSX_SCAN_STEP(op, "2")        \
+    GSX_SCAN_STEP(op, "4")                                             \
+    op " %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf\n\t"          \
+    op " %1, %1, %1 row_shr:8 row_mask:0xf bank_mask:0xf"
+__device__ __forceinline__ void row_scan_mul(float& a, float& b) {
+    asm volatile(GSX_SCAN("v_mul_f32_dpp") : "+v"(a), "+v"(b));
+}
+__device__ __forceinline__ void row_scan_add(float& a, float& b) {
+    asm volatile(GSX_SCAN("v_add_f32_dpp") : "+v"(a), "+v"(b));
+}
+
+// The wave's pixels.  The lanes 4 b .. 4 b + 3 of row r hold T and Q of step
+// 4 b + k in registers k: a step reads them with a row broadcast folded into
+// the consuming instruction and writes them with one DPP move under a bank
+// mask (in LDS, two 16-byte reads per pair of steps made the LDS the bound:
+// 66 % of the cycles).
+struct BwdPixels {
+    float T[4], Q[4];
+    int nc;        // n_contrib of step l % 16, row l / 16
+    float px[8];   // the columns' centres (scalar registers)
+};
+
+// A wave-uniform float in a scalar register (the compiler keeps one that
+// vector instructions computed in a vector register).  The lane read needs a
+// wait state after the VALU write of its operand and a VALU read of its
+// result two, neither of which the compiler's hazard check sees.
+__device__ __forceinline__ float scalar_float(float v) {
+    float s;
+    asm("s_nop 0\n\tv_readfirstlane_b32 %0, %1\n\ts_nop 1" : "=s"(s) : "v"(v));
+    return s;
+}
+
+template <int LANE>
+__device__ __forceinline__ int row_bcast(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x150 + LANE, 0xF, 0xF, true);  // row_newbcast
+}
+template <int LANE>
+__device__ __forceinline__ float row_bcast(float v) {
+    return __int_as_float(row_bcast<LANE>(__float_as_int(v)));
+}
+// old, with the lanes of bank B (4 B .. 4 B + 3 of each row) set to the row's lane 15 of v
+template <int B>
+__device__ __forceinline__ float set_bank(float old, float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v),
+                                                       0x150 + 15, 0xF, 1 << B, false));
+}
+// the quad's lane K in its four lanes
+template <int K>
+__device__ __forceinline__ float quad_bcast(float v) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(v), K * 0x55, 0xF, 0xF, true));
+}
+
+// The quadrant's cotangents in the two operand layouts.
+template <int CHP>
+struct BwdCot {
+    // A operand of c . g, per group of 4 x 4 pixels
+    float a[BwdShape<CHP>::kNarrow ? 1 : 4][BwdShape<CHP>::KS];
+    // A operand of dL/dc, per step
+    float b[BwdShape<CHP>::kNarrow ? 1 : 16][BwdShape<CHP>::CB];
+};
+
+// The wave's buffered entries, backmost first, and its other pieces of LDS.
+struct BwdLds {
+    float4* r0;   // mean x, mean y, log-alpha bound, opacity
+    float4* r1;   // -a/2, -b, -c/2 (conic), Gaussian id (int bits)
+    int* k;       // position in the tile's list
+    float* g;     // the pixels' cotangents, rows of CHP (BwdShape::kNarrow)
+    float* out;   // a bucket's gradients, rows of NO (6 geometric, then channels)
+    int* id;      // its Gaussians (-1: none)
+};
+
+// The lane's index from the execution hardware, opaque to the compiler.
+__device__ __forceinline__ int lane_again() {
+    uint32_t z = 0;
+    asm volatile("" : "+s"(z));
+    return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, z));
+}
+
+// One bucket: the entries b0 .. b0 + 15 of the buffer, of which those below cnt
+// are real.  PLAIN: every one passed plain_gaussian and the quadrant's
+// cotangents are finite; an entry that a pixel does not composite then runs
+// the same arithmetic with alpha = h = 0, and h carries the opacity
+// (h = o G dL/dalpha).  FIN: features and cotangents are finite, so the
+// matrix cores may multiply them by zero weights; otherwise the channel work
+// is done pair by pair and only where a pixel composites the Gaussian.
+// next: called before the gradients are reduced, to issue the loads that
+// follow the bucket.  The gradients stay in LDS until bwd_send.
+template <int CHP, bool PLAIN, bool FIN, class Next>
+__device__ __forceinline__ void bwd_bucket(const BwdLds& L, int b0, int cnt, BwdPixels& P,
+                                           const BwdCot<CHP>& g,
+                                           const float (&fb)[BwdShape<CHP>::KS],
+                                           const BwdOut& O, const float* __restrict__ gout,
+                                           const float* __restrict__ feat, int qx0, int qy0, int W,
+                                           int H, Next&& next) {
+    using S = BwdShape<CHP>;
+    const int lane = lane_again();  // the bucket's forms share no registers derived from it
+    const int j = lane & 15, r = lane >> 4, C = O.C;
+    const float py0 = (float)(qy0 + r) + 0.5f, py1 = (float)(qy0 + 4 + r) + 0.5f;
+    {
+        const float4 r0 = L.r0[b0 + j], r1 = L.r1[b0 + j];
+        const int k = L.k[b0 + j];
+        // the columns whose pixels (any of eight) composited past the
+        // bucket's frontmost entry
+        const int front = __builtin_amdgcn_readfirstlane(L.k[min(b0 + kBucket, cnt) - 1]);
+        uint64_t live = __ballot(P.nc > front);
+        live |= live >> 32;
+        live |= live >> 16;
+        const uint32_t cols = (uint32_t)(live | (live >> 8)) & 0xFFu;
+        const float dya = r0.y - py0, dyb = r0.y - py1;
+        const float cya = (r1.z * dya) * dya, cyb = (r1.z * dyb) * dyb;
+        float ha0 = 0.0f, ha1 = 0.0f, ha2 = 0.0f, hb0 = 0.0f, hb1 = 0.0f, hb2 = 0.0f;
+        mx_floatx4 dc[S::CB];
+#pragma unroll
+        for (int cb = 0; cb < S::CB; ++cb) dc[cb] = mx_floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+
+        // A operand of c . g for group q (columns 4 (q & 1).., rows 4 (q >> 1)..)
+        auto cota = [&](int q, int ks) {
+            if constexpr (S::kNarrow)
+                return L.g[(4 * (4 * (q & 1) + (j & 3) + 8 * (q >> 1)) + (j >> 2)) * CHP +
+                           4 * ks + r];
+            else
+                return g.a[q][ks];
+        };
+        // A operand of dL/dc at step s
+        auto cot = [&](int s, int cb) {
+            if constexpr (S::kNarrow)
+                return L.g[(4 * s + r) * CHP + (j & (CHP - 1))];
+            else
+                return g.b[s][cb];
+        };
+        // cotangent of channel c of the lane's pixel at step s (a pixel outside
+        // the image has no contributor)
+        auto pix = [&](int s, int c) {
+            int rr = r;  // opaque: no step's address is kept in registers
+            asm volatile("" : "+v"(rr));
+            if constexpr (S::kNarrow)
+                return L.g[(4 * s + rr) * CHP + c];
+            else
+                return gout[((int64_t)min(qy0 + 4 * (s >> 3) + rr, H - 1) * W +
+                             min(qx0 + (s & 7), W - 1)) * C + c];
+        };
+        // column x: steps x (row group a) and x + 8 (b)
+        auto column = [&](auto xc, float cga, float cgb) {
+            constexpr int x = decltype(xc)::value, K = x & 3, B = x >> 2;
+            const float dx = r0.x - P.px[x];
+            const float adx = r1.x * dx;
+            // splat_power with the products of dx alone and dy alone shared
+            const float pa = fmaf(fmaf(r1.y, dya, adx), dx, cya);
+            const float pb = fmaf(fmaf(r1.y, dyb, adx), dx, cyb);
+            const float Ga = PLAIN ? splat_exp_core(pa) : splat_exp_sel(pa);
+            const float Gb = PLAIN ? splat_exp_core(pb) : splat_exp_sel(pb);
+            const float oa = r0.w * Ga, ob = r0.w * Gb;
+            // min(0.99, o G) < 1/255 exactly when o G < 1/255
+            uint64_t ma = __ballot(k < row_bcast<x>(P.nc)) & __ballot(!(pa < r0.z)) &
+                          __ballot(!(oa < 1.0f / 255.0f));
+            uint64_t mb = __ballot(k < row_bcast<x + 8>(P.nc)) & __ballot(!(pb < r0.z)) &
+                          __ballot(!(ob < 1.0f / 255.0f));
+            if (!PLAIN) {
+                ma &= __ballot(!(pa > 0.0f));
+                mb &= __ballot(!(pb > 0.0f));
+            }
+            const bool ka = __builtin_amdgcn_inverse_ballot_w64(ma);
+            const bool kb = __builtin_amdgcn_inverse_ballot_w64(mb);
+            const float va = ka ? (PLAIN ? oa : fminf(0.99f, oa)) : 0.0f;
+            const float vb = kb ? (PLAIN ? ob : fminf(0.99f, ob)) : 0.0f;
+            const float ala = PLAIN ? fminf(0.99f, va) : va;
+            const float alb = PLAIN ? fminf(0.99f, vb) : vb;
+            const float ra = __builtin_amdgcn_rcpf(1.0f - ala);
+            const float rb = __builtin_amdgcn_rcpf(1.0f - alb);
+            float Ta = ra, Tb = rb;
+            row_scan_mul(Ta, Tb);
+            Ta *= row_bcast<4 * B>(P.T[K]);
+            Tb *= row_bcast<4 * B + 8>(P.T[K]);
+            const float wa = ala * Ta, wb = alb * Tb;
+            if (!FIN) {
+                // c . g pair by pair
+                cga = cgb = 0.0f;
+#pragma unroll 1
+                for (int c = 0; c < O.nc; ++c) {
+                    const float fc = feat[(int64_t)max(__float_as_int(r1.w), 0) * C + c];
+                    cga = fmaf(fc, pix(x, c), cga);
+                    cgb = fmaf(fc, pix(x + 8, c), cgb);
+                }
+            }
+            const float xa = (PLAIN || ka) ? wa * cga : 0.0f, xb = (PLAIN || kb) ? wb * cgb : 0.0f;
+            float Qa = xa, Qb = xb;
+            row_scan_add(Qa, Qb);
+            Qa += row_bcast<4 * B>(P.Q[K]);
+            Qb += row_bcast<4 * B + 8>(P.Q[K]);
+            // the frontmost entry's lane carries the pixel on
+            P.T[K] = set_bank<B>(P.T[K], Ta);
+            P.T[K] = set_bank<B + 2>(P.T[K], Tb);
+            P.Q[K] = set_bank<B>(P.Q[K], Qa);
+            P.Q[K] = set_bank<B + 2>(P.Q[K], Qb);
+            const float da = fmaf(cga, Ta, -((Qa - xa) * ra));
+            const float db = fmaf(cgb, Tb, -((Qb - xb) * rb));
+            const float ha = PLAIN ? va * da : (ka ? Ga * da : 0.0f);
+            const float hb = PLAIN ? vb * db : (kb ? Gb * db : 0.0f);
+            const float dx2 = dx * dx;
+            ha0 += ha;
+            hb0 += hb;
+            if (PLAIN) {
+                ha1 = fmaf(ha, dx, ha1);
+                hb1 = fmaf(hb, dx, hb1);
+                ha2 = fmaf(ha, dx2, ha2);
+                hb2 = fmaf(hb, dx2, hb2);
+            } else {
+                // an infinite offset of an entry that is not composited must not enter
+                ha1 = ka ? fmaf(ha, dx, ha1) : ha1;
+                hb1 = kb ? fmaf(hb, dx, hb1) : hb1;
+                ha2 = ka ? fmaf(ha, dx2, ha2) : ha2;
+                hb2 = kb ? fmaf(hb, dx2, hb2) : hb2;
+            }
+            if (FIN) {
+#pragma unroll
+                for (int cb = 0; cb < S::CB; ++cb) {
+                    // rows channels, columns entries
+                    dc[cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(cot(x, cb), wa, dc[cb], 0, 0, 0);
+                    dc[cb] =
+                        __builtin_amdgcn_mfma_f32_16x16x4f32(cot(x + 8, cb), wb, dc[cb], 0, 0, 0);
+                }
+            } else if (ka || kb) {
+                float* const dst = O.feat + O.feat_stride * __float_as_int(r1.w);
+#pragma unroll 1
+                for (int c = 0; c < O.nc; ++c)
+                    atomicAdd(dst + c, (ka ? wa * pix(x, c) : 0.0f) +
+                                           (kb ? wb * pix(x + 8, c) : 0.0f));
+            }
+        };
+        // a 4-column half: its c . g products, then its columns
+        auto half = [&](auto gxc) {
+            constexpr int gx = decltype(gxc)::value;
+            if (((cols >> (4 * gx)) & 15u) == 0u) return;
+            mx_floatx4 ca = {0.0f, 0.0f, 0.0f, 0.0f}, cc = {0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (FIN) {
+#pragma unroll
+                for (int ks = 0; ks < S::KS; ++ks) {
+                    ca = __builtin_amdgcn_mfma_f32_16x16x4f32(cota(gx, ks), fb[ks], ca, 0, 0, 0);
+                    cc = __builtin_amdgcn_mfma_f32_16x16x4f32(cota(gx + 2, ks), fb[ks], cc, 0, 0,
+                                                              0);
+                }
+            }
+            if ((cols >> (4 * gx)) & 1u) column(Int<4 * gx>{}, ca[0], cc[0]);
+            if ((cols >> (4 * gx)) & 2u) column(Int<4 * gx + 1>{}, ca[1], cc[1]);
+            if ((cols >> (4 * gx)) & 4u) column(Int<4 * gx + 2>{}, ca[2], cc[2]);
+            if ((cols >> (4 * gx)) & 8u) column(Int<4 * gx + 3>{}, ca[3], cc[3]);
+        };
+        half(Int<0>{});
+        half(Int<1>{});
+        next();
+
+        // the moments over the lane's two rows, as the reference's gradients
+        // (rasterize.py:197-218, dL/dG = o dL/dalpha; the staged conic is
+        // (-a/2, -b, -c/2)), then summed over the wave's four: row r of the
+        // wave ends with values row_value(r) and 4 + row_value(r)
+        const float ya = PLAIN || ha0 != 0.0f || ha1 != 0.0f ? dya : 0.0f;
+        const float yb = PLAIN || hb0 != 0.0f || hb1 != 0.0f ? dyb : 0.0f;
+        const float s0 = ha0 + hb0, sx = ha1 + hb1, sy = fmaf(ha0, ya, hb0 * yb);
+        const float o = PLAIN ? 1.0f : r0.w;
+        float v[8], h[4], q[2];
+        v[0] = 2.0f * r1.x * sx + r1.y * sy;
+        v[1] = r1.y * sx + 2.0f * r1.z * sy;
+        v[2] = -0.5f * (ha2 + hb2);
+        v[3] = -fmaf(ha1, ya, hb1 * yb);
+        v[4] = -0.5f * fmaf(ha0 * ya, ya, (hb0 * yb) * yb);
+        v[5] = PLAIN ? (s0 != 0.0f ? s0 / r0.w : 0.0f) : s0;
+        v[6] = v[7] = 0.0f;
+        if (!PLAIN) {
+#pragma unroll
+            for (int i = 0; i < 5; ++i) v[i] = (s0 != 0.0f || v[i] != 0.0f) ? o * v[i] : 0.0f;
+        }
+        reduce_step1<0, 3, 8, 6>(v, h);
+        h[3] = 0.0f;
+        reduce_step2<0, 2, 8>(h, q);
+        const int rv = row_value(r);
+        float* const row = L.out + j * S::NO;
+        row[rv] = q[0];
+        if (rv < 2) row[4 + rv] = q[1];
+#pragma unroll
+        for (int cb = 0; cb < S::CB; ++cb) {
+            // dc: channels 16 cb + 4 r + i of entry j (sent pair by pair if not FIN)
+            if (16 * cb + 4 * r < CHP) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) row[6 + 16 * cb + 4 * r + i] = FIN ? dc[cb][i] : 0.0f;
+            }
+        }
+        if (r == 0) L.id[j] = __float_as_int(r1.w);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    }
+}
+
+// The atomics of the bucket whose gradients lie in LDS.  An instruction's lanes
+// take whole entries, component by component: the atomics execute at 20.4 G
+// 64-byte lines/s whatever a line holds (measured, random and neighbouring
+// lines alike), so an entry's components go out together and lie in as few
+// lines as possible.  Memory operations complete in order, and a load issued
+// behind atomics waits for them too: the caller sends a bucket's gradients
+// once the loads of the next bucket have arrived, so that they drain under
+// its arithmetic.
+template <int CHP>
+__device__ __forceinline__ void bwd_send(const BwdLds& L, const BwdOut& O) {
+    using S = BwdShape<CHP>;
+    const int lane = lane_again();
+    auto part = [&](int first, int count, int per, int mul, float* base, int64_t stride) {
+        const int e0 = (int)((uint32_t)(lane * mul) >> 16), c = lane - e0 * count;
+        if (e0 >= per) return;
+        for (int e = e0; e < kBucket; e += per) {
+            const float val = L.out[e * S::NO + first + c];
+            const int64_t id = L.id[e];
+            if (id >= 0 && val != 0.0f) {
+                float* dst = base + stride * id + c;
+                if (first == 0 && !O.record)
+                    dst = c < 2   ? O.xy + 2 * id + c
+                          : c < 5 ? O.conic + 3 * id + (c - 2)
+                                  : O.opac + id;
+                atomicAdd(dst, val);
+            }
+        }
+    };
+    if (O.whole) {
+        part(0, 6 + O.nc, O.per, O.mul, O.xy, O.stride);
+    } else {
+        part(0, 6, 10, 65536 / 6 + 1, O.xy, O.stride);
+        part(6, O.nc, O.per, O.mul, O.feat, O.feat_stride);
+    }
+    // the next bucket's gradients overwrite these
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+}
+
+constexpr float kTame = 1e15f;  // 32 products of two below it stay far inside float
+
+constexpr int bwd_wide_waves(int chp) { return chp == 8 ? 5 : (chp == 16 ? 4 : 3); }
+
+// One wave per quadrant, with no barrier and nothing shared between the
+// quadrants of a tile: the wave reads the tile's list backmost first in
+// chunks of 64, keeps the Gaussians that can reach its quadrant in a buffer
+// in LDS (compacted, so every bucket but the last is full) and replays the
+// buffer 16 entries at a time.  A needed list entry reaches 1.0 to 1.5 of a
+// tile's four quadrants (1.06 with 1M Gaussians at 1080p), so summing the
+// quadrants' gradients before the atomics would save little, while batches
+// shared by the four waves cost four barriers each and leave 16 % of the
+// bucket lanes empty (32 channels: 367 us, against 283 us).
+template <int CHP>
+__global__ __launch_bounds__(kWave, bwd_wide_waves(CHP)) void k_raster_bwd_wide(
+    const float2* __restrict__ xy, const float4* __restrict__ co, const float* __restrict__ feat,
+    int C, int c0, int nc, const int* __restrict__ ids, const int2* __restrict__ ranges,
+    int64_t n, int64_t n_ids, const float* __restrict__ bg, int W, int H, int tiles_x, int slots,
+    const float* __restrict__ final_T, const int* __restrict__ n_contrib,
+    const float* __restrict__ grad_out, const float* __restrict__ grad_T,
+    float* __restrict__ g_xy, float* __restrict__ g_conic, float* __restrict__ g_feat,
+    float* __restrict__ g_opac, int gstride, const int* __restrict__ order) {
+    using S = BwdShape<CHP>;
+    constexpr int GS = CHP < 16 ? CHP : 16;
+    // wide blocks' cotangents pass through the records' space, 16 channels of
+    // 64 pixels at a time, before the first entries are buffered
+    constexpr int kRec = 9 * S::BUF;
+    constexpr int kBuf = S::kNarrow || kRec >= kWave * GS ? kRec : kWave * GS;
+    __shared__ __align__(16) float s_buf[kBuf];
+    __shared__ __align__(16) float s_g[S::kNarrow ? kWave * CHP : 4];
+    __shared__ __align__(16) float s_out[kBucket * S::NO];
+    __shared__ int s_id[kBucket];
+    const BwdLds L{reinterpret_cast<float4*>(s_buf), reinterpret_cast<float4*>(s_buf) + S::BUF,
+                   reinterpret_cast<int*>(s_buf + 8 * S::BUF), s_g, s_out, s_id};
+
+    // workgroups 32 i + 8 q + x: quadrant q of the tile in slot 8 i + x, so
+    // a tile's quadrants run on one XCD close together
+    const uint32_t bid = blockIdx.x;
+    const int slot = (int)((bid & 7u) | ((bid >> 5) << 3)), quad = (int)(bid >> 3) & 3;
+    if (slot >= slots) return;
+    const int tile = __builtin_amdgcn_readfirstlane(tile_at(order, slot, slots, true));
+    if (tile < 0) return;  // past the end of this XCD's band
+    const int tx = tile % tiles_x, ty = tile / tiles_x;
+    const int qx0 = tx * kTile + (quad & 1) * 8, qy0 = ty * kTile + (quad >> 1) * 8;
+    const float* const gout = grad_out + c0;
+
+    int start, num;
+    tile_span(ranges[tile], n_ids, start, num);
+    start = __builtin_amdgcn_readfirstlane(start);
+    num = __builtin_amdgcn_readfirstlane(num);
+
+    // the lane's own pixel (step lane % 16, row lane / 16): T and Q behind
+    // the list's end and its contributor count
+    BwdPixels P;
+    BwdCot<CHP> g;
+    bool fin = true;
+    int top;  // list entries not read yet; later ones changed no pixel
+    {
+        const int lane = threadIdx.x, j = lane & 15, r = lane >> 4;
+        const int opx = qx0 + (j & 7), opy = qy0 + 4 * (j >> 3) + r;
+        const bool inside = opx < W && opy < H;
+        // the pixel's loads issue together (clamped indices, masked after)
+        const int64_t pid = inside ? (int64_t)opy * W + opx : 0;
+        const float tf = final_T[pid];
+        const int nct = n_contrib[pid];
+        const float gt = grad_T ? grad_T[pid] : 0.0f;
+        P.nc = inside ? nct : 0;
+        int m = P.nc;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, kWave));
+        top = min(__builtin_amdgcn_readfirstlane(m), num);
+        if (top <= 0) return;
+        // the quadrant's cotangents, from the lanes that own the pixels into
+        // the operand layouts (zero outside the image or the block)
+        float bg_dot = 0.0f;
+        float* const buf = S::kNarrow ? s_g : s_buf;
+#pragma unroll
+        for (int cb = 0; cb < S::CB; ++cb) {
+#pragma unroll
+            for (int q = 0; q < GS; q += 4) {
+                float v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int ch = 16 * cb + q + i;
+                    v[i] = (inside && ch < nc) ? gout[pid * C + min(ch, nc - 1)] : 0.0f;
+                    fin = fin && fabsf(v[i]) < kTame;
+                    if (bg && ch < nc) bg_dot = bg_dot + bg[c0 + ch] * v[i];
+                }
+                *reinterpret_cast<float4*>(buf + (4 * j + r) * GS + q) =
+                    make_float4(v[0], v[1], v[2], v[3]);
+            }
+            // the wave's LDS accesses complete in order; the fence keeps the
+            // compiler from moving the reads above the writes
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            if constexpr (!S::kNarrow) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int s = 4 * (q & 1) + (j & 3) + 8 * (q >> 1);
+#pragma unroll
+                    for (int ks = 0; ks < GS / 4; ++ks)
+                        g.a[q][4 * cb + ks] = buf[(4 * s + (j >> 2)) * GS + 4 * ks + r];
+                }
+#pragma unroll
+                for (int s = 0; s < 16; ++s) g.b[s][cb] = buf[(4 * s + r) * GS + j];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        }
+        // The alpha output's cotangent enters once, with the first channel block.
+        if (c0 == 0 && grad_T) bg_dot = bg_dot + gt;
+        const float T = inside ? tf : 1.0f, Q = inside ? tf * bg_dot : 0.0f;
+        fin = fin && fabsf(T) < 1e30f && fabsf(Q) < 1e30f;
+        P.T[0] = quad_bcast<0>(T);
+        P.T[1] = quad_bcast<1>(T);
+        P.T[2] = quad_bcast<2>(T);
+        P.T[3] = quad_bcast<3>(T);
+        P.Q[0] = quad_bcast<0>(Q);
+        P.Q[1] = quad_bcast<1>(Q);
+        P.Q[2] = quad_bcast<2>(Q);
+        P.Q[3] = quad_bcast<3>(Q);
+#pragma unroll
+        for (int x = 0; x < 8; ++x) P.px[x] = scalar_float((float)(qx0 + x) + 0.5f);
+    }
+    // No channel or cotangent so far reaches kTame: no c . g, and so no Q that a
+    // pixel carries on, is infinite.  Once one does, every later bucket masks
+    // each pair, for an infinite Q must not meet a weight of zero.
+    bool tame = __ballot(!fin) == 0ull;
+    BwdOut O;
+    O.record = gstride > 0;
+    O.xy = g_xy;
+    O.conic = g_conic;
+    O.opac = g_opac;
+    O.feat = g_feat ? g_feat + c0 : g_xy + 6 + c0;
+    O.feat_stride = g_feat ? C : gstride;
+    O.stride = gstride;
+    O.nc = nc;
+    O.C = C;
+    // a block's channels follow the geometric gradients in its record
+    O.whole = O.record && !g_feat && c0 == 0;
+    const int comps = O.whole ? 6 + nc : nc;
+    O.per = kWave / comps;
+    O.mul = 65536 / comps + 1;
+
+    // the next 64 list entries, backmost first: the lane's Gaussian (-1: none)
+    // and its record and channels
+    auto load_id = [&]() {
+        const int k = top - 1 - lane_again();
+        int id = -1;
+        if (k >= 0) id = ids[start + k];
+        return (uint32_t)id < (uint64_t)n ? id : -1;
+    };
+    int id = -1;
+    float2 m;
+    float4 c;
+    auto load_record = [&]() {
+        const int64_t at = max(id, 0);
+        m = xy[at];
+        c = co[at];
+    };
+    id = load_id();
+    load_record();
+
+    int cnt = 0;             // buffered entries
+    bool all_plain = true;   // every one of them is plain
+    bool pending = false;    // a bucket's gradients wait in LDS
+    do {
+        // buffer those that reach the quadrant
+        {
+            const int lane = lane_again();
+            const bool keep = id >= 0 && quadrant_reached(m.x, m.y, c, qx0, qy0);
+            const uint64_t kept = __ballot(keep);
+            bool plain = true;
+            if (keep) {
+                const float thr = alpha_floor_power(c.w);
+                const int at = cnt + __popcll(kept & ((1ull << lane) - 1ull));
+                L.r0[at] = make_float4(m.x, m.y, thr, c.w);
+                L.r1[at] = make_float4(-0.5f * c.x, -c.y, -0.5f * c.z, __int_as_float(id));
+                L.k[at] = top - 1 - lane;
+                plain = plain_gaussian<0>(m.x, m.y, c, thr, nullptr);
+            }
+            all_plain = (cnt == 0 || all_plain) && __ballot(!plain) == 0ull;
+            cnt += __popcll(kept);
+            top -= kWave;
+        }
+        const bool end = top <= 0;
+        const int used = end ? cnt : cnt & ~(kBucket - 1);
+        if (end && (cnt & (kBucket - 1)) != 0) {
+            // fill the last bucket with records no pixel can take (alpha bound
+            // +inf)
+            const int at = cnt + lane_again();
+            if (at < ((cnt + kBucket - 1) & ~(kBucket - 1))) {
+                L.r0[at] = make_float4(0.0f, 0.0f, __builtin_huge_valf(), 0.0f);
+                L.r1[at] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(-1));
+                L.k[at] = 0x7fffffff;
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        if (!end) id = load_id();
+        if (!end && used == 0) load_record();
+#pragma unroll 1
+        for (int b0 = 0; b0 < used; b0 += kBucket) {
+            const int lane = lane_again(), j = lane & 15, r = lane >> 4;
+            // the next entries' records are loaded by the chunk's last bucket
+            const bool fetch = !end && b0 + kBucket >= used;
+            auto next = [&]() {
+                if (fetch) {
+                    load_record();
+                } else {  // not read; no register holds a value over the bucket
+                    asm volatile("" : "=v"(m.x), "=v"(m.y), "=v"(c.x), "=v"(c.y), "=v"(c.z),
+                                      "=v"(c.w));
+                }
+            };
+            // the entry's channels 4 ks + r, the B operand of c . g
+            float fb[S::KS];
+            bool ffin = true;
+            {
+                const float* const fp =
+                    feat + (int64_t)max(__float_as_int(L.r1[b0 + j].w), 0) * C + c0;
+#pragma unroll
+                for (int ks = 0; ks < S::KS; ++ks) fb[ks] = fp[min(4 * ks + r, nc - 1)];
+#pragma unroll
+                for (int ks = 0; ks < S::KS; ++ks) {
+                    fb[ks] = 4 * ks + r < nc ? fb[ks] : 0.0f;
+                    ffin = ffin && fabsf(fb[ks]) < kTame;
+                }
+            }
+            tame = tame && __ballot(!ffin) == 0ull;
+            if (pending) bwd_send<CHP>(L, O);
+            pending = true;
+            const float* const ft = feat + c0;
+            if (tame && all_plain)
+                bwd_bucket<CHP, true, true>(L, b0, cnt, P, g, fb, O, gout, ft, qx0, qy0, W, H,
+                                            next);
+            else if (tame)
+                bwd_bucket<CHP, false, true>(L, b0, cnt, P, g, fb, O, gout, ft, qx0, qy0, W, H,
+                                            next);
+            else
+                bwd_bucket<CHP, false, false>(L, b0, cnt, P, g, fb, O, gout, ft, qx0, qy0, W, H,
+                                            next);
+        }
+        if (end) break;
+        // the entries left over move to the front
+        if (used > 0) {
+            const int j = lane_again(), left = cnt - used;
+            if (j < left) {
+                const float4 a = L.r0[used + j], b = L.r1[used + j];
+                const int k = L.k[used + j];
+                L.r0[j] = a;
+                L.r1[j] = b;
+                L.k[j] = k;
+            }
+            cnt = left;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        }
+    } while (true);
+    if (pending) bwd_send<CHP>(L, O);
 }
 
 // Matrix-core forward for 32-channel blocks.  The per-pixel loop keeps every
@@ -2024,8 +2114,9 @@ __global__ __launch_bounds__(kOrderThreads) void k_tile_order(const int2* __rest
     tile_order_band<BWD>(blockIdx.x, ranges, work, n_ids, tiles, order, s_order);
 }
 
-// The gradient outputs to clear: one record (a, na floats, 16-byte aligned,
-// na a multiple of 4) or four arrays.
+// The gradient outputs to clear: one record (p[0], n[0] floats, 16-byte
+// aligned, n[0] a multiple of 4) and perhaps the features' array (p[2]), or
+// four arrays.
 struct ZeroGrads {
     float* p[4];
     int64_t n[4];
@@ -2052,11 +2143,30 @@ __global__ __launch_bounds__(kOrderThreads) void k_bwd_prologue(ZeroGrads z, int
         float4* a = reinterpret_cast<float4*>(z.p[0]);
         for (int64_t i = b * kOrderThreads + threadIdx.x; i < z.n[0] / 4; i += stride)
             a[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        return;
+        z.n[0] = 0;
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r)
         for (int64_t i = b * kOrderThreads + threadIdx.x; i < z.n[r]; i += stride) z.p[r][i] = 0.0f;
+}
+
+// The geometric part of a gradient record as separate arrays, a lane per
+// Gaussian: 32 bytes read (the record's first two 16-byte pieces) and 24
+// written; bound by the launch (5 us at 200k Gaussians, which the record
+// saves many times over in the backward's atomics).
+__global__ __launch_bounds__(256) void k_split_grads(int64_t n, const float* __restrict__ rec,
+                                                     int stride, float2* __restrict__ g_xy,
+                                                     float* __restrict__ g_conic,
+                                                     float* __restrict__ g_opac) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const float4* const r = reinterpret_cast<const float4*>(rec + i * stride);
+    const float4 a = r[0], b = r[1];
+    g_xy[i] = make_float2(a.x, a.y);
+    g_conic[3 * i] = a.z;
+    g_conic[3 * i + 1] = a.w;
+    g_conic[3 * i + 2] = b.x;
+    g_opac[i] = b.y;
 }
 
 int pick_ch(int nc) {
@@ -2097,23 +2207,105 @@ void launch_fwd(dim3 grid, hipStream_t st, bool depth, const float2* xy, const f
 }
 
 template <int CH>
-void launch_bwd(dim3 grid, hipStream_t st, const float2* xy, const float4* co, const float* feat,
+void launch_bwd(int slots, hipStream_t st, const float2* xy, const float4* co, const float* feat,
                 int C, int c0, int nc, const int* ids, const int2* ranges, int64_t n,
                 int64_t n_ids, const float* bg, int W, int H, int tiles_x, const float* fT,
                 const int* ncon, const float* gout, const float* gT, float* gxy, float* gcon,
                 float* gfeat, float* gop, int gstride, const int* order) {
-    if constexpr (CH == 32)
-        hipLaunchKernelGGL((k_raster_bwd_mx<CH>), grid, dim3(kThreads), 0, st, xy, co, feat, C,
-                           c0, nc, ids, ranges, n, n_ids, bg, W, H, tiles_x, fT, ncon, gout, gT,
-                           gxy, gcon, gfeat, gop, gstride, order);
+    if constexpr (CH > 4)
+        // four quadrant workgroups per tile slot, slots in groups of eight (XCDs)
+        hipLaunchKernelGGL((k_raster_bwd_wide<CH>), dim3(32u * (((unsigned)slots + 7u) / 8u)),
+                           dim3(kWave), 0, st, xy, co, feat, C, c0, nc, ids, ranges, n, n_ids, bg,
+                           W, H, tiles_x, slots, fT, ncon, gout, gT, gxy, gcon, gfeat, gop,
+                           gstride, order);
     else
-        hipLaunchKernelGGL((k_raster_bwd<CH>), grid, dim3(kThreads), 0, st, xy, co, feat, C, c0,
-                           nc, ids, ranges, n, n_ids, bg, W, H, tiles_x, fT, ncon, gout, gT, gxy,
-                           gcon, gfeat, gop, gstride, order);
+        hipLaunchKernelGGL((k_raster_bwd<CH>), dim3((unsigned)slots), dim3(kThreads), 0, st, xy,
+                           co, feat, C, c0, nc, ids, ranges, n, n_ids, bg, W, H, tiles_x, fT,
+                           ncon, gout, gT, gxy, gcon, gfeat, gop, gstride, order);
 }
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 inline bool aligned8(const void* p) { return ((uintptr_t)p & 7u) == 0; }
+
+// The backward into the outputs the two entry points accept.
+int raster_bwd(int64_t n, int32_t C, const float* means2d, const float* conic_opacity,
+                   const float* features, const int32_t* sorted_ids, int64_t num_ids,
+                   const int32_t* tile_ranges,
+                   const float* background, int32_t width, int32_t height, const float* final_T,
+                   const int32_t* n_contrib, const float* grad_out, const float* grad_final_T,
+                   float* g_means2d, float* g_conics, float* g_features, float* g_opacities,
+                   int32_t grad_stride, int32_t* tile_order, void* stream) {
+    if (n < 0 || num_ids < 0 || C <= 0 || width <= 0 || height <= 0) return GSX_ERR_INVALID;
+    if (!tile_ranges || !final_T || !n_contrib || !grad_out) return GSX_ERR_INVALID;
+    const bool rec = grad_stride > 0;
+    if (n > 0 && (!means2d || !conic_opacity || !features || !g_means2d ||
+                  (!rec && (!g_conics || !g_features || !g_opacities))))
+        return GSX_ERR_INVALID;
+    if (num_ids > 0 && !sorted_ids) return GSX_ERR_INVALID;
+    if (!aligned8(means2d) || !aligned16(conic_opacity) || !aligned8(tile_ranges))
+        return GSX_ERR_INVALID;
+    hipStream_t st = (hipStream_t)stream;
+    if (n == 0) return GSX_OK;
+    const int tiles_x = (width + kTile - 1) / kTile;
+    const int tiles_y = (height + kTile - 1) / kTile;
+    const int tiles = tiles_x * tiles_y;
+    // tile_order: [0, T) the forward's bounds, [T, T + 16 ceil(T / 8)) this
+    // call's order, one entry per workgroup
+    int* const order = tile_order ? tile_order + tiles : nullptr;
+    const int slots = order ? (int)(tile_order_words(tiles) - tiles) : tiles;
+    {
+        // gradient clearing and the tile order in one launch
+        ZeroGrads z{};
+        z.record = rec;
+        if (rec) {
+            z.p[0] = g_means2d;
+            z.n[0] = (int64_t)grad_stride * n;
+            z.p[2] = g_features;
+            z.n[2] = g_features ? (int64_t)C * n : 0;
+        } else {
+            z.p[0] = g_means2d;
+            z.n[0] = 2 * n;
+            z.p[1] = g_conics;
+            z.n[1] = 3 * n;
+            z.p[2] = g_features;
+            z.n[2] = (int64_t)C * n;
+            z.p[3] = g_opacities;
+            z.n[3] = n;
+        }
+        const int64_t most =
+            rec ? std::max(z.n[0] / 4, z.n[2]) : std::max<int64_t>((int64_t)C, 3) * n;
+        const int bands = order ? kOrderBands : 0;
+        const unsigned blocks =
+            (unsigned)std::min<int64_t>((most + kOrderThreads - 1) / kOrderThreads, 2048);
+        hipLaunchKernelGGL(k_bwd_prologue, dim3(blocks + (unsigned)bands), dim3(kOrderThreads), 0,
+                           st, z, bands, (const int*)tile_order, num_ids, tiles, order);
+        GSX_LAUNCH_CHECK();
+    }
+    for (int c0 = 0; c0 < C; c0 += kMaxChunk) {
+        const int nc = (C - c0 < kMaxChunk) ? C - c0 : kMaxChunk;
+        switch (pick_ch(nc)) {
+#define GSX_BWD_CASE(V)                                                                          \
+    case V:                                                                                      \
+        launch_bwd<V>(slots, st, (const float2*)means2d, (const float4*)conic_opacity, features, \
+                      C, c0, nc, sorted_ids, (const int2*)tile_ranges, n, num_ids, background,   \
+                      width, height, tiles_x, final_T, n_contrib, grad_out, grad_final_T,        \
+                      g_means2d, g_conics, g_features, g_opacities, grad_stride, order);         \
+        break;
+            GSX_BWD_CASE(1)
+            GSX_BWD_CASE(2)
+            GSX_BWD_CASE(3)
+            GSX_BWD_CASE(4)
+            GSX_BWD_CASE(8)
+            GSX_BWD_CASE(16)
+            GSX_BWD_CASE(32)
+#undef GSX_BWD_CASE
+            default:
+                return GSX_ERR_INVALID;
+        }
+        GSX_LAUNCH_CHECK();
+    }
+    return GSX_OK;
+}
 
 }  // namespace
 
@@ -2184,81 +2376,48 @@ int64_t gsx_tile_order_words(int32_t width, int32_t height) {
 
 int gsx_raster_bwd(int64_t n, int32_t C, const float* means2d, const float* conic_opacity,
                    const float* features, const int32_t* sorted_ids, int64_t num_ids,
-                   const int32_t* tile_ranges,
-                   const float* background, int32_t width, int32_t height, const float* final_T,
-                   const int32_t* n_contrib, const float* grad_out, const float* grad_final_T,
-                   float* g_means2d, float* g_conics, float* g_features, float* g_opacities,
-                   int32_t grad_stride, int32_t* tile_order, void* stream) {
-    if (n < 0 || num_ids < 0 || C <= 0 || width <= 0 || height <= 0) return GSX_ERR_INVALID;
-    if (!tile_ranges || !final_T || !n_contrib || !grad_out) return GSX_ERR_INVALID;
+                   const int32_t* tile_ranges, const float* background, int32_t width,
+                   int32_t height, const float* final_T, const int32_t* n_contrib,
+                   const float* grad_out, const float* grad_final_T, float* g_means2d,
+                   float* g_conics, float* g_features, float* g_opacities, int32_t grad_stride,
+                   int32_t* tile_order, void* stream) {
     const bool rec = grad_stride > 0;
     if (grad_stride < 0 || (rec && (grad_stride % 4 != 0 || grad_stride < 6 + C ||
                                     !aligned16(g_means2d) || g_conics || g_features ||
                                     g_opacities)))
         return GSX_ERR_INVALID;
-    if (n > 0 && (!means2d || !conic_opacity || !features || !g_means2d ||
-                  (!rec && (!g_conics || !g_features || !g_opacities))))
-        return GSX_ERR_INVALID;
-    if (num_ids > 0 && !sorted_ids) return GSX_ERR_INVALID;
-    if (!aligned8(means2d) || !aligned16(conic_opacity) || !aligned8(tile_ranges))
-        return GSX_ERR_INVALID;
-    hipStream_t st = (hipStream_t)stream;
+    return raster_bwd(n, C, means2d, conic_opacity, features, sorted_ids, num_ids, tile_ranges,
+                      background, width, height, final_T, n_contrib, grad_out, grad_final_T,
+                      g_means2d, g_conics, g_features, g_opacities, grad_stride, tile_order,
+                      stream);
+}
+
+int gsx_raster_bwd_geometry(int64_t n, int32_t C, const float* means2d, const float* conic_opacity,
+                            const float* features, const int32_t* sorted_ids, int64_t num_ids,
+                            const int32_t* tile_ranges, const float* background, int32_t width,
+                            int32_t height, const float* final_T, const int32_t* n_contrib,
+                            const float* grad_out, const float* grad_final_T, float* g_geometry,
+                            float* g_features, int32_t grad_stride, int32_t* tile_order,
+                            void* stream) {
+    if (grad_stride < 8 || grad_stride % 4 != 0 || !aligned16(g_geometry)) return GSX_ERR_INVALID;
+    if (n > 0 && !g_features) return GSX_ERR_INVALID;
+    return raster_bwd(n, C, means2d, conic_opacity, features, sorted_ids, num_ids, tile_ranges,
+                      background, width, height, final_T, n_contrib, grad_out, grad_final_T,
+                      g_geometry, nullptr, g_features, nullptr, grad_stride, tile_order, stream);
+}
+
+int gsx_split_raster_grads(int64_t n, const float* record, int32_t grad_stride, float* g_means2d,
+                           float* g_conics, float* g_opacities, void* stream) {
+    if (n < 0 || grad_stride < 8 || grad_stride % 4 != 0) return GSX_ERR_INVALID;
     if (n == 0) return GSX_OK;
-    const int tiles_x = (width + kTile - 1) / kTile;
-    const int tiles_y = (height + kTile - 1) / kTile;
-    const int tiles = tiles_x * tiles_y;
-    // tile_order: [0, T) the forward's bounds, [T, T + 16 ceil(T / 8)) this
-    // call's order, one entry per workgroup
-    int* const order = tile_order ? tile_order + tiles : nullptr;
-    const dim3 grid((unsigned)(order ? tile_order_words(tiles) - tiles : tiles));
-    {
-        // gradient clearing and the tile order in one launch
-        ZeroGrads z{};
-        z.record = rec;
-        if (rec) {
-            z.p[0] = g_means2d;
-            z.n[0] = (int64_t)grad_stride * n;
-        } else {
-            z.p[0] = g_means2d;
-            z.n[0] = 2 * n;
-            z.p[1] = g_conics;
-            z.n[1] = 3 * n;
-            z.p[2] = g_features;
-            z.n[2] = (int64_t)C * n;
-            z.p[3] = g_opacities;
-            z.n[3] = n;
-        }
-        const int64_t most = rec ? z.n[0] / 4 : std::max<int64_t>((int64_t)C, 3) * n;
-        const int bands = order ? kOrderBands : 0;
-        const unsigned blocks =
-            (unsigned)std::min<int64_t>((most + kOrderThreads - 1) / kOrderThreads, 2048);
-        hipLaunchKernelGGL(k_bwd_prologue, dim3(blocks + (unsigned)bands), dim3(kOrderThreads), 0,
-                           st, z, bands, (const int*)tile_order, num_ids, tiles, order);
-        GSX_LAUNCH_CHECK();
-    }
-    for (int c0 = 0; c0 < C; c0 += kMaxChunk) {
-        const int nc = (C - c0 < kMaxChunk) ? C - c0 : kMaxChunk;
-        switch (pick_ch(nc)) {
-#define GSX_BWD_CASE(V)                                                                          \
-    case V:                                                                                      \
-        launch_bwd<V>(grid, st, (const float2*)means2d, (const float4*)conic_opacity, features,  \
-                      C, c0, nc, sorted_ids, (const int2*)tile_ranges, n, num_ids, background,   \
-                      width, height, tiles_x, final_T, n_contrib, grad_out, grad_final_T,        \
-                      g_means2d, g_conics, g_features, g_opacities, grad_stride, order);         \
-        break;
-            GSX_BWD_CASE(1)
-            GSX_BWD_CASE(2)
-            GSX_BWD_CASE(3)
-            GSX_BWD_CASE(4)
-            GSX_BWD_CASE(8)
-            GSX_BWD_CASE(16)
-            GSX_BWD_CASE(32)
-#undef GSX_BWD_CASE
-            default:
-                return GSX_ERR_INVALID;
-        }
-        GSX_LAUNCH_CHECK();
-    }
+    if (!record || !g_means2d || !g_conics || !g_opacities || !aligned16(record) ||
+        !aligned8(g_means2d))
+        return GSX_ERR_INVALID;
+    const int64_t blocks = (n + 255) / 256;
+    if (blocks > 0x7fffffff) return GSX_ERR_TOO_LARGE;
+    hipLaunchKernelGGL(k_split_grads, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, n,
+                       record, (int)grad_stride, (float2*)g_means2d, g_conics, g_opacities);
+    GSX_LAUNCH_CHECK();
     return GSX_OK;
 }
 

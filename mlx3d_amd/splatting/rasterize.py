@@ -116,6 +116,41 @@ def raster_backward(means2d, conic_opac, feats, sorted_ids, tile_ranges, backgro
     return g_m, g_c, g_f, g_o
 
 
+def raster_backward_geometry(means2d, conic_opac, feats, sorted_ids, tile_ranges, background,
+                             width, height, final_T, n_contrib, g_out, g_final_T,
+                             tile_order=None):
+    """gsx_raster_bwd_geometry: (record (N, 8) = [means2d 2 | conic 3 | opacity
+    1 | padding], feature gradient (N, C)).  The geometric atomics of a Gaussian
+    share one cache line, which three arrays would spread over three."""
+    dev = means2d.device
+    n, C = feats.shape
+    rec = _empty((n, 8), dev)
+    g_f = _empty((n, C), dev)
+    if g_out is None:
+        g_out = torch.zeros((height, width, C), dtype=torch.float32, device=dev)
+    g_out = _lib.f32c(g_out)
+    g_final_T = None if g_final_T is None else _lib.f32c(g_final_T)
+    _lib.check(_lib.load().gsx_raster_bwd_geometry(
+        n, C, _lib.ptr(means2d), _lib.ptr(conic_opac), _lib.ptr(feats), _lib.ptr(sorted_ids),
+        sorted_ids.numel(), _lib.ptr(tile_ranges), _lib.ptr(background), width, height,
+        _lib.ptr(final_T), _lib.ptr(n_contrib), _lib.ptr(g_out), _lib.ptr(g_final_T),
+        _lib.ptr(rec), _lib.ptr(g_f), 8, _lib.ptr(tile_order), _lib.stream_handle(dev)),
+        "gsx_raster_bwd_geometry")
+    return rec, g_f
+
+
+def split_geometry(rec):
+    """(means2d (N, 2), conics (N, 3), opacities (N,)) of a geometry record."""
+    dev = rec.device
+    n = rec.shape[0]
+    g_m, g_c, g_o = _empty((n, 2), dev), _empty((n, 3), dev), _empty((n,), dev)
+    _lib.check(_lib.load().gsx_split_raster_grads(n, _lib.ptr(rec), rec.shape[1], _lib.ptr(g_m),
+                                                  _lib.ptr(g_c), _lib.ptr(g_o),
+                                                  _lib.stream_handle(dev)),
+               "gsx_split_raster_grads")
+    return g_m, g_c, g_o
+
+
 def pack_conic_opacity(conics, opacities):
     dev = conics.device
     n = conics.shape[0]
@@ -147,9 +182,10 @@ class _Rasterize(torch.autograd.Function):
     def backward(ctx, g_out, g_final_T, g_alpha, _g_nc):
         means2d, co, feats, ids, ranges, bg, final_T, n_contrib, order = ctx.saved_tensors
         width, height = ctx.size
-        g_m, g_c, g_f, g_o = raster_backward(means2d, co, feats, ids, ranges, bg, width, height,
-                                             final_T, n_contrib, g_out,
-                                             t_cotangent(g_final_T, g_alpha), tile_order=order)
+        rec, g_f = raster_backward_geometry(means2d, co, feats, ids, ranges, bg, width, height,
+                                            final_T, n_contrib, g_out,
+                                            t_cotangent(g_final_T, g_alpha), tile_order=order)
+        g_m, g_c, g_o = split_geometry(rec)
         return g_m, g_c, g_f, g_o, None, None, None, None, None
 
 

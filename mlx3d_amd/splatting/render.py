@@ -23,8 +23,8 @@ import torch
 from .. import _lib
 from ..cameras import Camera
 from ..profiling import count, stage
-from .rasterize import (background_tensor, raster_backward, raster_forward, t_cotangent,
-                        tile_order_buffer)
+from .rasterize import (background_tensor, raster_backward, raster_backward_geometry,
+                        raster_forward, t_cotangent, tile_order_buffer)
 from .sh import num_sh_bases
 from .tiles import BinJob
 
@@ -139,21 +139,19 @@ class _RenderFn(torch.autograd.Function):
         # The rasterizer's gradients go into one record per Gaussian, which
         # the screen statistics and the preprocess VJP read in place.  A
         # feature render hands its feature gradient to autograd instead: a
-        # strided view of the record would be copied there, so it takes the
-        # four-array layout (a contiguous (N, C) feature gradient).
+        # strided view of the record would be copied there, so its record
+        # holds the geometric gradients only.
         record = bool(cfg.sh_mode) or cfg.adam is not None
+        args = (means2d, co, feats, ids, ranges, background, cfg.width, cfg.height, final_T,
+                n_contrib, g_image, t_cotangent(g_final_T, g_alpha))
         with stage("raster_bwd"):
-            r = raster_backward(
-                means2d, co, feats, ids, ranges, background, cfg.width, cfg.height, final_T,
-                n_contrib, g_image, t_cotangent(g_final_T, g_alpha), record=record,
-                tile_order=order)
-        if record:
-            _, _, g_feat, _, grec, gstride = r
-            g_in = (grec, None, None)  # g_means2d (the record), g_conics, g_opac_eff
-        else:
-            g_m2r, g_con, g_feat, g_op = r
-            gstride = 0
-            g_in = (g_m2r, g_con, g_op)
+            if record:
+                _, _, g_feat, _, grec, gstride = raster_backward(*args, record=True,
+                                                                 tile_order=order)
+            else:
+                grec, g_feat = raster_backward_geometry(*args, tile_order=order)
+                gstride = grec.shape[1]
+        g_in = (grec, None, None)  # g_means2d (the record), g_conics, g_opac_eff
         if cfg.screen_stats is not None:
             acc, cnt = cfg.screen_stats
             _lib.check(_lib.load().gsx_accum_screen_grads(

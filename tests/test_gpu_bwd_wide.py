@@ -1,0 +1,90 @@
+"""The backward for five channels and more (lanes are Gaussians): list lengths
+around its buckets (16), its chunks (64) and its buffer (80), partial tiles and
+quadrants, every channel block, non-finite inputs, and the geometry record with
+its split form, against the oracle."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import cu, host, say
+from mlx3d_amd.splatting import bin_gaussians
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(n, C, W, H, seed):
+    """n 2D Gaussians that all reach every tile of a small image; every 40th
+    is a needle (conic past the plain bound), opacities from faint to 1."""
+    rng = np.random.default_rng(seed)
+    m2 = np.stack([rng.uniform(-2, W + 2, n), rng.uniform(-2, H + 2, n)], 1).astype(np.float32)
+    a, c = rng.uniform(0.005, 0.2, n), rng.uniform(0.005, 0.2, n)
+    b = rng.uniform(-0.8, 0.8, n) * np.sqrt(a * c)
+    a[::40], c[::40], b[::40] = 1e3, 1e-4, 0.0
+    con = np.stack([a, b, c], 1).astype(np.float32)
+    op = rng.uniform(0.003, 1.0, n).astype(np.float32)
+    op[op < 0.3] *= 0.1  # long lists before a pixel stops
+    feats = rng.standard_normal((n, C)).astype(np.float32)
+    depths = rng.uniform(1, 2, n).astype(np.float32)
+    radii = np.full(n, 64.0, np.float32)
+    ids, ranges, _, _ = bin_gaussians(cu(m2), cu(radii), cu(depths), W, H)
+    return m2, con, op, feats, ids, ranges, rng
+
+
+def _both(m2, con, op, feats, ids, ranges, W, H, bg, g_img, g_T):
+    from mlx3d_amd.splatting.rasterize import (pack_conic_opacity, raster_backward_geometry,
+                                               raster_forward, split_geometry)
+
+    ref = O.raster_fwd(m2, con, op, feats, host(ids), host(ranges), W, H, bg=bg)
+    rg = O.raster_bwd(m2, con, op, feats, host(ids), host(ranges), W, H, ref["final_T"],
+                      ref["n_contrib"], g_img, grad_final_T=g_T, bg=bg)
+    co = pack_conic_opacity(cu(con), cu(op))
+    _, fT, nc, _, _ = raster_forward(cu(m2), co, cu(feats), ids, ranges, cu(bg), W, H)
+    np.testing.assert_array_equal(host(nc), ref["n_contrib"])
+    rec, gf = raster_backward_geometry(cu(m2), co, cu(feats), ids, ranges, cu(bg), W, H, fT, nc,
+                                       cu(g_img), cu(g_T))
+    gm, gc, go = split_geometry(rec)
+    got = {"means2d": gm, "conics": gc, "opacities": go, "features": gf}
+    assert float(rec[:, 6:].abs().max()) == 0.0
+    return {k: (host(v), np.asarray(rg[k])) for k, v in got.items()}
+
+
+@pytest.mark.parametrize("n,C,W,H", [(1, 5, 1, 1), (15, 8, 23, 9), (16, 9, 16, 16),
+                                     (17, 16, 7, 23), (79, 17, 23, 9), (80, 32, 17, 15),
+                                     (81, 5, 33, 8), (400, 12, 23, 9), (400, 37, 16, 17)])
+def test_wide_backward_list_edges(n, C, W, H):
+    m2, con, op, feats, ids, ranges, rng = _scene(n, C, W, H, 100 + n + C)
+    bg = rng.random(C, dtype=np.float32)
+    g_img = rng.standard_normal((H, W, C)).astype(np.float32)
+    g_T = rng.standard_normal((H, W)).astype(np.float32)
+    # A pixel's T is recovered entry by entry, each step a reciprocal (1 ulp)
+    # and a product: over L entries the relative error is below 2 L 2^-23, the
+    # largest list here has 400 (9.6e-5); sums over <= 561 pixels add less.
+    for k, (a, b) in _both(m2, con, op, feats, ids, ranges, W, H, bg, g_img, g_T).items():
+        e = float(np.abs(a - b).max() / (np.abs(b).max() + 1e-30))
+        say(f"  n={n} C={C} {W}x{H} {k}: {e:.2e}")
+        assert e < 1e-4, k
+
+
+@pytest.mark.parametrize("C", [6, 32])
+def test_wide_backward_non_finite(C):
+    """An infinite feature and a NaN cotangent reach exactly the gradients
+    that composite with them."""
+    W, H, n = 23, 9, 60
+    m2, con, op, feats, ids, ranges, rng = _scene(n, C, W, H, 7 + C)
+    con[:, [0, 2]] += 0.3  # small footprints: most pairs do not meet
+    feats[20, 1] = np.inf
+    g_img = rng.standard_normal((H, W, C)).astype(np.float32)
+    g_img[4, 11, C - 1] = np.nan
+    bg = np.zeros(C, np.float32)
+    g_T = np.zeros((H, W), np.float32)
+    for k, (a, b) in _both(m2, con, op, feats, ids, ranges, W, H, bg, g_img, g_T).items():
+        fin = np.isfinite(b)
+        say(f"  C={C} {k}: {int((~fin).sum())} of {fin.size} non-finite")
+        np.testing.assert_array_equal(np.isfinite(a), fin, err_msg=k)
+        assert fin.any()
+        e = float(np.abs(a[fin] - b[fin]).max() / (np.abs(b[fin]).max() + 1e-30))
+        assert e < 1e-4, k
