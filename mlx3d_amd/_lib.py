@@ -229,13 +229,17 @@ def check(status: int, what: str) -> int:
 
 
 def ptr(t: torch.Tensor | None):
-    if t is None:
-        return None
-    return ctypes.c_void_p(t.data_ptr())
+    """A tensor's address as the pointer argument of a C call."""
+    return None if t is None else t.data_ptr()
 
 
 def stream_handle(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """torch's current stream on `device`, without building a Stream object
+    (5 us, in every one of a pass's seven calls; the handle alone takes 0.3)."""
+    index = device.index
+    if index is None:
+        index = torch.cuda.current_device()
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(index))
 
 
 def require_device(*tensors: torch.Tensor | None) -> torch.device:

@@ -58,20 +58,28 @@ class StageTimer:
         self.counters[name].append(float(value))
 
 
-@contextlib.contextmanager
+class _Stage:
+    """A pair of events around a stage, kept by the active timer."""
+
+    def __init__(self, timer: StageTimer, name: str):
+        self._timer, self._name = timer, name
+
+    def __enter__(self):
+        self._a = torch.cuda.Event(enable_timing=True)
+        self._b = torch.cuda.Event(enable_timing=True)
+        self._a.record()
+
+    def __exit__(self, *exc):
+        self._b.record()
+        self._timer._pending.append((self._name, self._a, self._b))
+        return False
+
+
+_IDLE = contextlib.nullcontext()
+
+
 def stage(name: str):
-    t = _active
-    if t is None:
-        yield
-        return
-    a = torch.cuda.Event(enable_timing=True)
-    b = torch.cuda.Event(enable_timing=True)
-    a.record()
-    try:
-        yield
-    finally:
-        b.record()
-        t._pending.append((name, a, b))
+    return _IDLE if _active is None else _Stage(_active, name)
 
 
 def count(name: str, value: float):

@@ -43,11 +43,11 @@ def raster_forward(means2d, conic_opac, feats, sorted_ids, tile_ranges, backgrou
     ``order_ready``: the binning already wrote this frame's order there."""
     dev = means2d.device
     n, C = feats.shape
-    out = _empty((height, width, C), dev)
-    final_T = _empty((height, width), dev)
-    alpha = _empty((height, width), dev)
-    n_contrib = _empty((height, width), dev, torch.int32)
-    depth_map = _empty((height, width), dev) if depths is not None else None
+    f = means2d.new_empty
+    out = f(height, width, C)
+    final_T, alpha = f(height, width), f(height, width)
+    n_contrib = sorted_ids.new_empty(height, width)
+    depth_map = f(height, width) if depths is not None else None
     L = _lib.load()
     _lib.check(L.gsx_raster_fwd(n, C, _lib.ptr(means2d), _lib.ptr(conic_opac), _lib.ptr(feats),
                                 _lib.ptr(depths), _lib.ptr(sorted_ids), sorted_ids.numel(),

@@ -67,10 +67,12 @@ def _sh_views(cfg: _Cfg, sh_a, sh_b):
 def _forward(cfg: _Cfg, means, quats, scales, opacities, sh_a, sh_b, colors, background):
     dev = means.device
     n = means.shape[0]
-    f = lambda *s: torch.empty(s, dtype=torch.float32, device=dev)  # noqa: E731
-    i = lambda *s: torch.empty(s, dtype=torch.int32, device=dev)  # noqa: E731
+    f = means.new_empty  # float32; new_empty takes half the host time of torch.empty
     means2d, depths, radii, comp, co = f(n, 2), f(n), f(n), f(n), f(n, 4)
     colors_out = f(n, 3) if cfg.sh_mode else None
+    # the binning's placement launch writes the forward's tile order too
+    order = tile_order_buffer(cfg.width, cfg.height, dev)
+    i = order.new_empty  # int32
     counts, dkeys, rects = i(n), i(n), i(n, 2)
     sh0, s0, shr, sr = _sh_views(cfg, sh_a, sh_b)
     L = _lib.load()
@@ -83,8 +85,6 @@ def _forward(cfg: _Cfg, means, quats, scales, opacities, sh_a, sh_b, colors, bac
             _lib.ptr(colors_out), _lib.ptr(counts), _lib.ptr(dkeys), _lib.ptr(rects), st),
             "gsx_preprocess_fwd")
     feats = colors_out if cfg.sh_mode else colors
-    # the binning's placement launch writes the forward's tile order too
-    order = tile_order_buffer(cfg.width, cfg.height, dev)
     with stage("binning"):
         job = BinJob(counts, dkeys, rects, cfg.width, cfg.height,
                      refine=(means2d, co) if cfg.refine else None, tile_order=order)
@@ -180,7 +180,7 @@ class _RenderFn(torch.autograd.Function):
                     "gsx_preprocess_bwd_adam")
             opt.commit()
             return None, None, None, None, None, None, None, None, None
-        f = lambda *s: torch.empty(s, dtype=torch.float32, device=dev)  # noqa: E731
+        f = means.new_empty
         g_means, g_quats, g_scales, g_opac = f(n, 3), f(n, 4), f(n, 3), f(n)
         g_sh_a = g_sh_b = None
         if cfg.sh_mode:

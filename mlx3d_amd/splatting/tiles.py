@@ -17,6 +17,7 @@ from __future__ import annotations
 
 import collections
 import ctypes
+import struct
 import threading
 import time
 import weakref
@@ -31,6 +32,7 @@ _BIN_ERR_OVERFLOW = 2  # gsx_bin_error
 _ERR_TOO_LARGE = -4    # gsx_status
 _ERR_DEVICE = -5
 _STATUS_WORDS = 8
+_STATUS = struct.Struct(f"{_STATUS_WORDS}Q")
 _WAIT_LIMIT_S = 120.0  # a device that never publishes is reported, not waited on forever
 _HINT_WINDOW = 16      # jobs whose duplicate counts size the next capacity guess
 
@@ -56,15 +58,15 @@ class _HostStatus:
     def wait(self, k: int, seq: int) -> tuple[np.ndarray, int]:
         """The words of target k once they carry `seq` or a later sequence
         number (kernels of one stream publish in order), and that number."""
-        w = self.words[_STATUS_WORDS * k:_STATUS_WORDS * (k + 1)]
+        at = 8 * _STATUS_WORDS * k
         t0 = None
         spins = 0
         while True:
-            v = w.copy()
-            tags = (v >> np.uint64(32)).astype(np.uint32)
-            ahead = (tags - np.uint32(seq)).astype(np.uint32)  # modular: >= seq
-            if (ahead < np.uint32(1 << 31)).all() and (tags == tags[0]).all():
-                return (v & np.uint64(0xFFFFFFFF)).astype(np.uint32), int(tags[0])
+            v = _STATUS.unpack_from(self.words, at)
+            tag = v[0] >> 32
+            # modular: >= seq, and the same on every word
+            if (tag - seq) & 0xFFFFFFFF < 1 << 31 and all(x >> 32 == tag for x in v):
+                return np.array([x & 0xFFFFFFFF for x in v], np.uint32), tag
             spins += 1
             if spins % 4096 == 0:
                 t0 = t0 or time.perf_counter()
