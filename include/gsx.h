@@ -302,7 +302,8 @@ int gsx_bin_sort_async(int64_t n, const uint32_t* tile_counts,
  * host_status != NULL (8 words) its last kernel writes the final status
  * there the same way.  tile_order: NULL, or the gsx_tile_order_words(W, H)
  * buffer of the frame's gsx_raster_fwd: the call writes the forward's tile
- * order for the ranges it produces into words [T, 2T) (the placement's
+ * order for the ranges it produces into words [T, 2T) and clears the
+ * bounds before them (the placement's
  * first workgroups compute it beside the placement; it is what
  * gsx_raster_fwd would compute), to be passed with order_ready = 1.
  *
@@ -363,7 +364,8 @@ int gsx_pack_conic_opacity(int64_t n, const float* conics,
  * its tiles by; words [T, 2T) the order the workgroups take the tiles in
  * (each XCD's contiguous band of tiles, longest lists first).  With
  * order_ready != 0 words [T, 2T) already hold that order, written by
- * gsx_bin_tiles_async for these ranges, and the call only reads them.  The
+ * gsx_bin_tiles_async for these ranges, which cleared words [0, T) too, and
+ * the call only reads the order.  The
  * outputs do not depend on the order.  The buffer has no counterpart in the
  * reference (whose Metal dispatch has no such control). */
 int gsx_raster_fwd(int64_t n, int32_t C, const float* means2d,

@@ -38,6 +38,9 @@ using namespace gsx;
 
 namespace {
 
+template <int V>
+using Int = std::integral_constant<int, V>;
+
 constexpr int kThreads = kTilePixels;
 constexpr int kWaves = kThreads / kWave;  // 4 quadrant waves
 
@@ -326,11 +329,24 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
 // Ordering the whole frame instead, heaviest first regardless of bands,
 // balanced as well but doubled the rasterizers' HBM traffic (1.05 GB per
 // C3 backward instead of 0.47: neighbouring tiles on different XCDs).
-// by_block: order is indexed by workgroup (the backward's layout), else by
-// xcd_remap position; -1 = no tile.
+// by_block: order is indexed by workgroup (the backward's layout, -1 = no
+// tile), else by xcd_remap position.  The forward does not know a tile's work
+// beforehand, and a scene's crowded region fills a few bands: the busiest
+// XCD had 1.4 to 1.5 times the mean work at 3600 to 4096 tiles.  Up to
+// kDealTiles tiles its workgroups therefore take the bands' lists in turns
+// of eight ranks, each XCD an eighth of every band: 106 -> 94 us (300k
+// through a fisheye, 4096 tiles), 267 -> 239 us (32 channels, 500k, 3600
+// tiles), 82 -> 80 us (200k, 2040 tiles).  With 8160 tiles of 1M and 3M
+// Gaussians the bands' work is even (1.06, 1.04) and the lost locality
+// shows, 177 -> 180 and 188 -> 195 us, so larger frames keep whole bands.
+constexpr uint32_t kDealTiles = 6144;
 __device__ __forceinline__ int tile_at(const int* order, uint32_t b, uint32_t nb, bool by_block) {
     if (!order) return (int)xcd_remap(b, nb);
-    return order[by_block ? b : xcd_remap(b, nb)];
+    if (by_block) return order[b];
+    if (nb > kDealTiles) return order[xcd_remap(b, nb)];
+    const uint32_t q = nb / 8u, r = nb % 8u, i = b / 8u, x = b % 8u;
+    const uint32_t band = i < q ? (x + (i >> 3)) & 7u : x;
+    return order[band * q + min(band, r) + i];
 }
 
 // The workgroup's largest contributor count (n_contrib) into work[tile]:
@@ -348,17 +364,26 @@ __device__ __forceinline__ void store_tile_work(int* work, int tile, int last, i
         work[tile] = max(max(s_wmax[0], s_wmax[1]), max(s_wmax[2], s_wmax[3]));
 }
 
+// The lane's index from the execution hardware, opaque to the compiler:
+// values derived from it are formed where they are used instead of being held
+// in registers over a whole loop.
+__device__ __forceinline__ int lane_again() {
+    uint32_t z = 0;
+    asm volatile("" : "+s"(z));
+    return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, z));
+}
+
 // A quadrant wave's walk list: the staged Gaussians whose bit is set in the
 // quadrant's NW mask words (loader wave lw, lane l <-> staged index
-// 64 lw + l), compacted in LDS as 32-bit record byte offsets (16 x index)
+// 64 lw + l), compacted in LDS as 32-bit record byte offsets (step x index)
 // so the walk is a counted loop over uniform offsets.  Built by the wave
 // itself after the workgroup barrier that publishes the masks; ascending
 // index order (REV: descending).  list[cnt .. cnt + PADS - 1] are set to
-// pad, a valid record offset, for the walks' look-ahead.  Returns cnt
+// record pad's offset, for the walks' look-ahead.  Returns cnt
 // (uniform).
 template <int NW, bool REV, int PADS = 2>
 __device__ __forceinline__ int build_list(const uint64_t* words, uint32_t* list, int lane,
-                                          int pad) {
+                                          int step, int pad) {
     int total = 0;
     const uint64_t below = (1ull << lane) - 1ull;
     const uint64_t above = lane == 63 ? 0ull : ~((2ull << lane) - 1ull);
@@ -367,10 +392,10 @@ __device__ __forceinline__ int build_list(const uint64_t* words, uint32_t* list,
         const int lw = REV ? NW - 1 - k : k;
         const uint64_t m = uniform64(words[lw]);
         if ((m >> lane) & 1ull)
-            list[total + __popcll(m & (REV ? above : below))] = (uint32_t)((lw * kWave + lane) * 16);
+            list[total + __popcll(m & (REV ? above : below))] = (uint32_t)((lw * kWave + lane) * step);
         total += __popcll(m);
     }
-    if (lane < PADS) list[total + lane] = (uint32_t)pad;
+    if (lane < PADS) list[total + lane] = (uint32_t)(pad * step);
     return total;
 }
 
@@ -398,121 +423,168 @@ __device__ __forceinline__ float comp4(const float4& v, int e) {
     return e == 0 ? v.x : (e == 1 ? v.y : (e == 2 ? v.z : v.w));
 }
 
+// The staged record of the forward's walk: r0 = (mean x, mean y, opacity,
+// value 0), r1 = (-a/2, -b, -c/2, value 1) and the values from 2 on, where
+// the values are the channels and then the depth.  The walk reads a record
+// for every pair of a wave and a Gaussian, and an LDS read costs two cycles
+// per register it fills, broadcast or not: a separate log-alpha bound, depth
+// and padded channels (12 registers) kept the LDS busy for 82 of the 91
+// million cycles in which a CU had work (1M Gaussians, 1080p), so a record
+// holds nothing the loop can do without: 177 -> 166 us there, 188 -> 179 us
+// with 3M.  A wave alone on its SIMD gains nothing from it (a crowded tile of
+// Gaussians in a blob at 690 tiles: 169 -> 178 us with 60k).
+template <int NV>
+struct FwdRec {
+    static constexpr int EX = NV > 2 ? NV - 2 : 0;
+    static constexpr int X4 = (EX + 3) / 4;
+    static constexpr int kStride = 8 + 4 * X4;  // floats
+    float4 r0, r1;
+    float x[4 * X4 + 1];
+    __device__ __forceinline__ float value(int i) const {
+        return i == 0 ? r0.w : (i == 1 ? r1.w : x[i - 2]);
+    }
+    // the byte offset is a multiple of the stride
+    __device__ __forceinline__ void load(const float* base, uint32_t off) {
+        const char* p = reinterpret_cast<const char*>(base) + off;
+        r0 = *reinterpret_cast<const float4*>(p);
+        r1 = *reinterpret_cast<const float4*>(p + 16);
+    }
+    __device__ __forceinline__ void load_values(const float* base, uint32_t off) {
+        const char* p = reinterpret_cast<const char*>(base) + off + 32;
+        if constexpr (EX == 1) {
+            x[0] = *reinterpret_cast<const float*>(p);
+        } else if constexpr (EX == 2) {
+            const float2 v = *reinterpret_cast<const float2*>(p);
+            x[0] = v.x;
+            x[1] = v.y;
+        } else if constexpr (EX > 2) {
+#pragma unroll
+            for (int k = 0; k < X4; ++k) {
+                const float4 v = reinterpret_cast<const float4*>(p)[k];
+                x[4 * k] = v.x;
+                x[4 * k + 1] = v.y;
+                x[4 * k + 2] = v.z;
+                x[4 * k + 3] = v.w;
+            }
+        }
+    }
+};
+
+// A lane's pixel in the front-to-back loop: its centre, transmittance, sums
+// and the record offset of the last Gaussian composited in this batch.
+template <int NV>
+struct FwdPixel {
+    float x, y;
+    float T;
+    float acc[NV];
+    int last_off;
+};
+
 // One (pixel, Gaussian) step of the front-to-back loop (rasterize.py:74-87):
-// lanes that do not composite keep their state.  PLAIN: the Gaussian passed
-// plain_gaussian(), so its power is never positive and exp needs no range
-// handling; the channel sums then run under the compositing lanes' exec
-// mask (a branch that no lane takes is skipped).  Otherwise every update is
-// a select.  The per-lane decisions are kept as wave masks (alive: the
-// pixel has not stopped): a ballot of one comparison is that comparison's
-// lane mask, the masks combine in scalar registers, and inverse_ballot
-// hands one back to the lanes as a select condition, so none of it costs
-// vector ALU work.
-template <int CH, bool DEPTH, bool PLAIN>
-__device__ __forceinline__ void fwd_pair(const float4& r0, const float4& r1,
-                                         const float4 (&fv)[(CH + 3) / 4], int off,
-                                         float pxf, float pyf, float& T, float* acc,
-                                         float& dacc, int& last_off, uint64_t& alive) {
-    const float dx = r0.x - pxf, dy = r0.y - pyf;
-    const float power = splat_power(r1.x, r1.y, r1.z, dx, dy);
-    const uint64_t live =
-        PLAIN ? alive & __ballot(!(power < r0.z))
-              : alive & __ballot(!(power > 0.0f)) & __ballot(!(power < r0.z));
+// lanes that do not composite keep their state.  PLAIN: the Gaussian passed plain_gaussian(),
+// so its power is never positive; powers below -86, where exp would need
+// range handling, lie under the alpha bound whatever the opacity
+// (plain_gaussian: the log-alpha bound is at least -86).  The updates then
+// run under the compositing lanes' exec mask (a branch that no lane takes is
+// skipped, and a move costs 2.4 cycles where a select costs 4.2).  Otherwise
+// the log-alpha bound is applied as it stands and every update is a select.
+// The per-lane decisions are kept as wave masks (alive: the pixel has not
+// stopped): a ballot of one comparison is that comparison's lane mask, the
+// masks combine in scalar registers, and inverse_ballot hands one back to
+// the lanes as a select condition, so none of it costs vector ALU work.
+template <int NV, bool PLAIN>
+__device__ __forceinline__ void fwd_pair(const FwdRec<NV>& g, int off, FwdPixel<NV>& px,
+                                         uint64_t& alive) {
+    const float power = splat_power(g.r1.x, g.r1.y, g.r1.z, g.r0.x - px.x, g.r0.y - px.y);
+    const uint64_t live = PLAIN ? alive & __ballot(!(power < -86.0f))
+                                : alive & __ballot(!(power > 0.0f)) &
+                                      __ballot(!(power < alpha_floor_power(g.r0.z)));
     const float e = PLAIN ? splat_exp_core(power) : splat_exp_sel(power);
-    const float alpha = fminf(0.99f, r0.w * e);
+    const float alpha = fminf(0.99f, g.r0.z * e);
     const uint64_t pass = live & __ballot(!(alpha < 1.0f / 255.0f));
-    const float next_T = T * (1.0f - alpha);
+    const float next_T = px.T * (1.0f - alpha);
     const uint64_t lt = __ballot(next_T < 1e-4f);
     alive &= ~(pass & lt);  // the reference's early stop
     const bool add = __builtin_amdgcn_inverse_ballot_w64(pass & ~lt);
     // acc += rgb * (alpha * T) (rasterize.py:84) as one fused multiply-add,
     // the contraction Metal's default fast-math applies to the reference
-    const float w = alpha * T;
+    const float w = alpha * px.T;
     if (PLAIN) {
-        T = add ? next_T : T;
-        last_off = add ? off : last_off;
+        px.T = add ? next_T : px.T;
+        px.last_off = add ? off : px.last_off;
         if (add) {
             // keeps the sums a branch (the compiler would turn them into
             // selects) and w computed before it
             asm volatile("" ::"v"(w) : "memory");
 #pragma unroll
-            for (int ch = 0; ch < CH; ++ch) acc[ch] = fmaf(comp4(fv[ch >> 2], ch & 3), w, acc[ch]);
-            if (DEPTH) dacc = fmaf(r1.w, w, dacc);
+            for (int i = 0; i < NV; ++i) px.acc[i] = fmaf(g.value(i), w, px.acc[i]);
         }
-        return;
     } else {
+        px.T = add ? next_T : px.T;
+        px.last_off = add ? off : px.last_off;
 #pragma unroll
-        for (int ch = 0; ch < CH; ++ch) {
-            const float a2 = fmaf(comp4(fv[ch >> 2], ch & 3), w, acc[ch]);
-            acc[ch] = add ? a2 : acc[ch];
-        }
-        if (DEPTH) {
-            const float d2 = fmaf(r1.w, w, dacc);
-            dacc = add ? d2 : dacc;
+        for (int i = 0; i < NV; ++i) {
+            const float a2 = fmaf(g.value(i), w, px.acc[i]);
+            px.acc[i] = add ? a2 : px.acc[i];
         }
     }
-    T = add ? next_T : T;
-    last_off = add ? off : last_off;
 }
 
 // Front-to-back walk of one quadrant wave over its list, four Gaussians per
-// round: each Gaussian's records (and, up to four channels, its channels)
-// are read while the one before it is evaluated, and list entries two
-// places ahead.  list[cnt .. cnt + 3] are the padding record, which no pixel
-// takes, so a round may run past the list's end (a stale entry is read only
-// as the next round's offsets and never used, since the round count ends
-// first).  The wave stops once its 64 pixels have terminated.  last_off gets
-// the offset of each pixel's last composited Gaussian of this batch.
-template <int CH, bool DEPTH, bool PLAIN>
-__device__ __forceinline__ void fwd_walk(const uint32_t* list, int cnt, const float4* s_r0,
-                                         const float4* s_r1, const float4 (*s_f)[(CH + 3) / 4],
-                                         float pxf, float pyf, float& T, float* acc, float& dacc,
-                                         int& last_off, uint64_t& alive) {
-    constexpr int F4 = (CH + 3) / 4;
-    // more channels are read just before their pair (registers)
-    constexpr bool kAhead = F4 == 1;
+// round: each Gaussian's record (up to four values past the first two) is
+// read while the one before it is evaluated, and list entries two places
+// ahead.  list[cnt .. cnt + 3] are the padding record, which no pixel takes,
+// so a round may run past the list's end (a stale entry is read only as the
+// next round's offsets and never used, since the round count ends first).
+// The wave stops once its 64 pixels have terminated.  last_off gets the
+// offset of each pixel's last composited Gaussian of this batch.
+template <int NV, bool PLAIN>
+__device__ __forceinline__ void fwd_walk(const uint32_t* list, int cnt, const float* rec,
+                                         FwdPixel<NV>& px, uint64_t& alive) {
+    using Rec = FwdRec<NV>;
+    // more values are read just before their pair (registers)
+    constexpr bool kAhead = Rec::X4 <= 1;
     if (cnt == 0) return;
-    const float4* sf = &s_f[0][0];
-    float4 fa[F4], fb[F4];
-    auto feat = [&](float4 (&f)[F4], int off) {
-#pragma unroll
-        for (int q = 0; q < F4; ++q) f[q] = (&rec_at(sf, off * F4))[q];
+    Rec a, b;
+    auto load = [&](Rec& g, uint32_t off) {
+        g.load(rec, off);
+        if (kAhead) g.load_values(rec, off);
     };
-    auto pair = [&](const float4& r0, const float4& r1, float4 (&f)[F4], int off) {
-        if (!kAhead) feat(f, off);
-        fwd_pair<CH, DEPTH, PLAIN>(r0, r1, f, off, pxf, pyf, T, acc, dacc, last_off, alive);
+    auto pair = [&](Rec& g, uint32_t off) {
+        if (!kAhead) g.load_values(rec, off);
+        fwd_pair<NV, PLAIN>(g, (int)off, px, alive);
     };
-    int oa = list[0], ob = list[1];
-    float4 a0 = rec_at(s_r0, oa), a1 = rec_at(s_r1, oa);
-    if (kAhead) feat(fa, oa);
+    if (!PLAIN) {  // rare: one copy of the long form, nothing read ahead
+#pragma unroll 1
+        for (int i = 0; i < cnt && alive != 0ull; ++i) {
+            const uint32_t o = list[i];
+            load(a, o);
+            pair(a, o);
+        }
+        return;
+    }
+    uint32_t oa = list[0], ob = list[1];
+    load(a, oa);
     for (int i = 0;; i += 4) {
-        const int nc = list[i + 2], nd = list[i + 3];
-        float4 b0 = rec_at(s_r0, ob), b1 = rec_at(s_r1, ob);
-        if (kAhead) feat(fb, ob);
-        pair(a0, a1, fa, oa);
-        a0 = rec_at(s_r0, nc);
-        a1 = rec_at(s_r1, nc);
-        if (kAhead) feat(fa, nc);
-        pair(b0, b1, fb, ob);
-        const int na = list[i + 4], nb = list[i + 5];
-        b0 = rec_at(s_r0, nd);
-        b1 = rec_at(s_r1, nd);
-        if (kAhead) feat(fb, nd);
-        pair(a0, a1, fa, nc);
-        a0 = rec_at(s_r0, na);
-        a1 = rec_at(s_r1, na);
-        if (kAhead) feat(fa, na);
-        pair(b0, b1, fb, nd);
+        const uint32_t nc = list[i + 2], nd = list[i + 3];
+        load(b, ob);
+        pair(a, oa);
+        load(a, nc);
+        pair(b, ob);
+        const uint32_t na = list[i + 4], nb = list[i + 5];
+        load(b, nd);
+        pair(a, nc);
+        load(a, na);
+        pair(b, nd);
         if (alive == 0ull || i + 4 >= cnt) return;
         oa = na;
         ob = nb;
     }
 }
 
-// Occupancy targets that the compiler meets without spilling: seven waves
-// per SIMD (<= 72 VGPRs) up to three channels (C3's forward 193.8 -> 190.4
-// us against six), six up to four, five up to eight.
-constexpr int fwd_min_waves(int ch) { return ch <= 3 ? 7 : (ch <= 4 ? 6 : (ch <= 8 ? 5 : 1)); }
+// Occupancy targets that the compiler meets without spilling: eight waves
+// per SIMD (<= 64 VGPRs) up to three channels, seven up to eight.
+constexpr int fwd_min_waves(int ch) { return ch <= 3 ? 8 : (ch <= 8 ? 7 : 4); }
 
 template <int CH, bool DEPTH>
 __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
@@ -522,12 +594,11 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
     int W, int H, int tiles_x, float* __restrict__ out, float* __restrict__ final_T,
     int* __restrict__ n_contrib, float* __restrict__ depth_out, float* __restrict__ alpha_out,
     const int* __restrict__ order, int* __restrict__ work) {
-    constexpr int F4 = (CH + 3) / 4;
-    // entry kThreads of the records is the walk lists' padding: a record no
-    // pixel can take (alpha bound +inf)
-    __shared__ float4 s_r0[kThreads + 1];     // mean x, mean y, log-alpha bound, opacity
-    __shared__ float4 s_r1[kThreads + 1];     // -a/2, -b, -c/2 (conic), depth
-    __shared__ float4 s_f[kThreads + 1][F4];  // channels, zero padded
+    constexpr int NV = CH + (DEPTH ? 1 : 0);
+    using Rec = FwdRec<NV>;
+    constexpr int RS = Rec::kStride;
+    // record kThreads is the lists' padding: opacity zero, which no pixel takes
+    __shared__ __align__(16) float s_rec[(kThreads + 1) * RS];
     __shared__ uint64_t s_mask[kWaves][kWaves];  // [quadrant][loader wave]
     __shared__ uint32_t s_list[kWaves][kThreads + 8];  // walk lists (+ look-ahead room)
     // one word per wave, written before a barrier and read by every thread
@@ -537,33 +608,31 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
     __shared__ __align__(16) uint32_t s_alive[kWaves];
     __shared__ __align__(16) uint32_t s_plain[kWaves];
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tile = __builtin_amdgcn_readfirstlane(tile_at(order, blockIdx.x, gridDim.x, false));
     const int tx = tile % tiles_x, ty = tile / tiles_x;
     const int px0 = tx * kTile, py0 = ty * kTile;
     const int px = px0 + (wave & 1) * 8 + (lane & 7);
     const int py = py0 + (wave >> 1) * 8 + (lane >> 3);
     const bool inside = px < W && py < H;
-    const float pxf = (float)px + 0.5f, pyf = (float)py + 0.5f;
 
     int start, num;
     tile_span(ranges[tile], n_ids, start, num);
 
-    float T = 1.0f, dacc = 0.0f;
-    float acc[CH];
+    FwdPixel<NV> p;
+    p.x = (float)px + 0.5f;
+    p.y = (float)py + 0.5f;
+    p.T = 1.0f;
 #pragma unroll
-    for (int k = 0; k < CH; ++k) acc[k] = 0.0f;
+    for (int i = 0; i < NV; ++i) p.acc[i] = 0.0f;
     int last = 0;
     uint64_t alive = __ballot(inside);  // the wave's pixels still compositing
     // the padding record (written before the first barrier)
-    if (tid == 0) {
-        s_r0[kThreads] = make_float4(0.0f, 0.0f, __builtin_huge_valf(), 0.0f);
-        s_r1[kThreads] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll
-        for (int q = 0; q < F4; ++q) s_f[kThreads][q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
+    if (tid < RS) s_rec[kThreads * RS + tid] = 0.0f;
 
     for (int base = 0; base < num; base += kThreads) {
+        const int lane = lane_again(), tid = wave * kWave + lane;
         if (lane == 0) s_alive[wave] = alive != 0ull;
         __syncthreads();
         const uint4 al = *reinterpret_cast<const uint4*>(s_alive);
@@ -577,13 +646,26 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
                 // the record, depth and feature loads issue together
                 const float2 m = xy[g];
                 const float4 c = co[g];
-                const float dz = DEPTH ? depths[g] : 0.0f;
-                stage_features<CH>(s_f[tid], feat + (int64_t)g * C + c0, nc);
+                float v[4 * Rec::X4 + 2];
+#pragma unroll
+                for (int i = 0; i < 4 * Rec::X4 + 2; ++i) v[i] = 0.0f;
+                const float* const f = feat + (int64_t)g * C + c0;
+#pragma unroll
+                for (int ch = 0; ch < CH; ++ch)
+                    if (nc >= CH || ch < nc) v[ch] = f[ch];
+                if (DEPTH) v[CH] = depths[g];
                 const float thr = alpha_floor_power(c.w);
-                s_r0[tid] = make_float4(m.x, m.y, thr, c.w);
-                s_r1[tid] = make_float4(-0.5f * c.x, -c.y, -0.5f * c.z, dz);
+                float4* const r = reinterpret_cast<float4*>(s_rec + tid * RS);
+                r[0] = make_float4(m.x, m.y, c.w, v[0]);
+                r[1] = make_float4(-0.5f * c.x, -c.y, -0.5f * c.z, v[1]);
+#pragma unroll
+                for (int i = 0; i < Rec::X4; ++i)
+                    r[2 + i] = make_float4(v[2 + 4 * i], v[3 + 4 * i], v[4 + 4 * i],
+                                           v[5 + 4 * i]);
                 qm = quadrant_mask(m.x, m.y, c, px0, py0);
-                plain = plain_gaussian<CH>(m.x, m.y, c, thr, s_f[tid]) && fabsf(dz) < 1e30f;
+                plain = plain_gaussian<0>(m.x, m.y, c, thr, nullptr);
+#pragma unroll
+                for (int i = 0; i < NV; ++i) plain = plain && fabsf(v[i]) < 1e30f;
             }
         }
 #pragma unroll
@@ -598,34 +680,244 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
         const bool batch_plain = (pl.x & pl.y & pl.z & pl.w) != 0u;
         if (alive == 0ull) continue;
         const int cnt =
-            build_list<kWaves, false, 4>(s_mask[wave], s_list[wave], lane, kThreads * 16);
-        int last_off = -1;
+            build_list<kWaves, false, 4>(s_mask[wave], s_list[wave], lane, 4 * RS, kThreads);
+        p.last_off = -1;
         if (batch_plain)
-            fwd_walk<CH, DEPTH, true>(s_list[wave], cnt, s_r0, s_r1, s_f, pxf, pyf, T, acc, dacc,
-                                      last_off, alive);
+            fwd_walk<NV, true>(s_list[wave], cnt, s_rec, p, alive);
         else
-            fwd_walk<CH, DEPTH, false>(s_list[wave], cnt, s_r0, s_r1, s_f, pxf, pyf, T, acc,
-                                       dacc, last_off, alive);
-        if (last_off >= 0) last = base + (last_off >> 4) + 1;
+            fwd_walk<NV, false>(s_list[wave], cnt, s_rec, p, alive);
+        if (p.last_off >= 0) last = base + (int)((uint32_t)p.last_off / (4u * RS)) + 1;
     }
     if (inside) {
         const int64_t pid = (int64_t)py * W + px;
+        const float T = p.T;
         float* o = out + pid * C + c0;
 #pragma unroll
         for (int ch = 0; ch < CH; ++ch)
-            if (ch < nc) o[ch] = acc[ch] + T * (bg ? bg[c0 + ch] : 0.0f);
+            if (ch < nc) o[ch] = p.acc[ch] + T * (bg ? bg[c0 + ch] : 0.0f);
         if (c0 == 0) {
             final_T[pid] = T;
             n_contrib[pid] = last;
             if (alpha_out) alpha_out[pid] = 1.0f - T;
             if (DEPTH) {
                 const float al = 1.0f - T;
-                depth_out[pid] = al > 1e-6f ? dacc / al : 0.0f;
+                depth_out[pid] = al > 1e-6f ? p.acc[CH] / al : 0.0f;
             }
         }
     }
     if (work) store_tile_work(work, tile, last, wave, lane);
 }
+
+// The forward of small frames.  One wave composites a quadrant's list serially
+// in k_raster_fwd, about 45 instructions an entry, and a wave alone on its
+// SIMD issues one every six cycles: the tile with the longest list bounds the
+// launch (1889 entries: 106 us of a 256 x 256 view, 86 us here).  Only the chain through
+// T is serial, so here a workgroup has one quadrant: three waves evaluate
+// alphas, 16 entries of a chunk of 48 each, into LDS (zero where the pixel
+// does not take the entry), while wave 0 composites the chunk before.  The
+// arithmetic of a pair is fwd_pair's, so every output has its bits: an alpha
+// of zero leaves T and the sums of a plain batch as they are.
+constexpr int kSplitWaves = 3;                    // evaluating waves
+constexpr int kSplitPart = 16;                    // entries of a chunk per wave
+constexpr int kSplitChunk = kSplitWaves * kSplitPart;
+constexpr int kSplitRead = 8;                     // entries composited per round of reads
+static_assert(kSplitPart % kSplitRead == 0, "a round lies in one wave's part");
+
+template <int CH, bool DEPTH>
+__global__ __launch_bounds__(kThreads) void k_raster_fwd_split(
+    const float2* __restrict__ xy, const float4* __restrict__ co, const float* __restrict__ feat,
+    int C, int nc, const float* __restrict__ depths, const int* __restrict__ ids,
+    const int2* __restrict__ ranges, int64_t n, int64_t n_ids, const float* __restrict__ bg,
+    int W, int H, int tiles_x, int tiles, float* __restrict__ out, float* __restrict__ final_T,
+    int* __restrict__ n_contrib, float* __restrict__ depth_out, float* __restrict__ alpha_out,
+    const int* __restrict__ order, int* __restrict__ work) {
+    constexpr int NV = CH + (DEPTH ? 1 : 0);
+    constexpr int V4 = (NV + 3) / 4;
+    static_assert(kThreads == (kSplitWaves + 1) * kWave, "one compositing wave");
+    // the batch's entries that reach the quadrant, in list order
+    __shared__ float4 s_r0[kThreads];       // mean x, mean y, opacity, list position (int bits)
+    __shared__ float4 s_r1[kThreads];       // -a/2, -b, -c/2, log-alpha bound
+    __shared__ float4 s_v[kThreads][V4];    // channels, then depth
+    __shared__ float s_alpha[2][kSplitChunk][kWave];
+    __shared__ int s_cnt[kWaves];
+    __shared__ uint32_t s_plain[kWaves];
+    // chunk c's word c & 1: every pixel has stopped.  Written before the
+    // chunk's barrier and read after it; the next write of the word follows
+    // the next chunk's barrier, which every reader has reached.
+    __shared__ uint32_t s_stop[2];
+
+    // workgroups 32 i + 8 q + x: quadrant q of the tile in slot 8 i + x
+    const uint32_t bid = blockIdx.x;
+    const int slot = (int)((bid & 7u) | ((bid >> 5) << 3)), quad = (int)(bid >> 3) & 3;
+    if (slot >= tiles) return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tile = __builtin_amdgcn_readfirstlane(tile_at(order, slot, tiles, false));
+    const int qx0 = (tile % tiles_x) * kTile + (quad & 1) * 8;
+    const int qy0 = (tile / tiles_x) * kTile + (quad >> 1) * 8;
+    const int px = qx0 + (lane & 7), py = qy0 + (lane >> 3);
+    const bool inside = px < W && py < H;
+    const float pxf = (float)px + 0.5f, pyf = (float)py + 0.5f;
+
+    int start, num;
+    tile_span(ranges[tile], n_ids, start, num);
+
+    // wave 0's pixels
+    float T = 1.0f, acc[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) acc[i] = 0.0f;
+    int last = 0;
+    uint64_t alive = __ballot(inside);
+
+    bool stopped = false;
+    for (int base = 0; base < num && !stopped; base += kThreads) {
+        const int k = base + tid;
+        bool keep = false, plain = true;
+        float2 m = make_float2(0.0f, 0.0f);
+        float4 c = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        float v[4 * V4], thr = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4 * V4; ++i) v[i] = 0.0f;
+        if (k < num) {
+            const int g = ids[start + k];
+            if ((uint32_t)g < (uint64_t)n) {
+                // the record, depth and feature loads issue together
+                m = xy[g];
+                c = co[g];
+                const float* const f = feat + (int64_t)g * C;
+#pragma unroll
+                for (int ch = 0; ch < CH; ++ch)
+                    if (nc >= CH || ch < nc) v[ch] = f[ch];
+                if (DEPTH) v[CH] = depths[g];
+                keep = quadrant_reached(m.x, m.y, c, qx0, qy0);
+                thr = alpha_floor_power(c.w);
+                plain = plain_gaussian<0>(m.x, m.y, c, thr, nullptr);
+#pragma unroll
+                for (int i = 0; i < NV; ++i) plain = plain && fabsf(v[i]) < 1e30f;
+            }
+        }
+        const uint64_t kept = __ballot(keep), odd = __ballot(keep && !plain);
+        if (lane == 0) {
+            s_cnt[wave] = __popcll(kept);
+            s_plain[wave] = odd == 0ull;
+        }
+        __syncthreads();
+        int cnt = 0, at = __popcll(kept & ((1ull << lane) - 1ull));
+        bool batch_plain = true;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            if (w < wave) at += s_cnt[w];
+            cnt += s_cnt[w];
+            batch_plain = batch_plain && s_plain[w] != 0u;
+        }
+        cnt = __builtin_amdgcn_readfirstlane(cnt);
+        if (keep) {
+            s_r0[at] = make_float4(m.x, m.y, c.w, __int_as_float(k));
+            s_r1[at] = make_float4(-0.5f * c.x, -c.y, -0.5f * c.z, thr);
+#pragma unroll
+            for (int i = 0; i < V4; ++i)
+                s_v[at][i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+        }
+        __syncthreads();
+        const int chunks = (cnt + kSplitChunk - 1) / kSplitChunk;
+        for (int ck = 0; ck <= chunks; ++ck) {
+            if (wave > 0) {
+                const int j0 = (wave - 1) * kSplitPart, e0 = ck * kSplitChunk + j0;
+                if (e0 < cnt) {
+#pragma unroll 4
+                    for (int j = 0; j < kSplitPart; ++j) {
+                        const int e = min(e0 + j, cnt - 1);  // past the end: alpha zero
+                        const float4 r0 = s_r0[e], r1 = s_r1[e];
+                        const float power =
+                            splat_power(r1.x, r1.y, r1.z, r0.x - pxf, r0.y - pyf);
+                        const bool ok = batch_plain ? !(power < -86.0f)
+                                                    : !(power > 0.0f) && !(power < r1.w);
+                        const float ex =
+                            batch_plain ? splat_exp_core(power) : splat_exp_sel(power);
+                        const float alpha = fminf(0.99f, r0.z * ex);
+                        const bool take = ok && !(alpha < 1.0f / 255.0f) && e0 + j < cnt;
+                        s_alpha[ck & 1][j0 + j][lane] = take ? alpha : 0.0f;
+                    }
+                }
+            } else {
+                if (ck > 0) {
+                    const int f0 = (ck - 1) * kSplitChunk;
+                    const int len = min(kSplitChunk, cnt - f0);
+                    const float(*const sa)[kWave] = s_alpha[(ck - 1) & 1];
+                    int at_last = -1;
+                    auto entry = [&](int j, float a, const float4* val, bool masked) {
+                        const float next_T = T * (1.0f - a);
+                        // the reference's early stop (a is zero, and next_T
+                        // the T of a living pixel, where the entry is not taken)
+                        alive &= ~__ballot(next_T < 1e-4f);
+                        const bool add = __builtin_amdgcn_inverse_ballot_w64(alive);
+                        const float w = add ? a * T : 0.0f;
+                        T = add ? next_T : T;
+                        at_last = w > 0.0f ? j : at_last;
+#pragma unroll
+                        for (int i = 0; i < NV; ++i) {
+                            const float s = fmaf(comp4(val[i >> 2], i & 3), w, acc[i]);
+                            acc[i] = (!masked || w > 0.0f) ? s : acc[i];
+                        }
+                    };
+                    if (batch_plain) {
+                        // eight at a time, their reads together; entries past
+                        // the end have alpha zero and the last one's values
+                        for (int j = 0; j < len; j += kSplitRead) {
+                            float a[kSplitRead];
+                            float4 val[kSplitRead][V4];
+#pragma unroll
+                            for (int u = 0; u < kSplitRead; ++u) {
+                                a[u] = sa[j + u][lane];
+#pragma unroll
+                                for (int i = 0; i < V4; ++i)
+                                    val[u][i] = s_v[min(f0 + j + u, cnt - 1)][i];
+                            }
+#pragma unroll
+                            for (int u = 0; u < kSplitRead; ++u)
+                                entry(j + u, a[u], val[u], false);
+                        }
+                    } else {
+#pragma unroll 1
+                        for (int j = 0; j < len; ++j) entry(j, sa[j][lane], s_v[f0 + j], true);
+                    }
+                    if (at_last >= 0) last = __float_as_int(s_r0[f0 + at_last].w) + 1;
+                }
+                if (lane == 0) s_stop[ck & 1] = alive == 0ull;
+            }
+            __syncthreads();
+            stopped = s_stop[ck & 1] != 0u;
+            if (stopped) break;
+        }
+    }
+    if (wave > 0) return;
+    if (inside) {
+        const int64_t pid = (int64_t)py * W + px;
+        float* o = out + pid * C;
+#pragma unroll
+        for (int ch = 0; ch < CH; ++ch)
+            if (ch < nc) o[ch] = acc[ch] + T * (bg ? bg[ch] : 0.0f);
+        final_T[pid] = T;
+        n_contrib[pid] = last;
+        if (alpha_out) alpha_out[pid] = 1.0f - T;
+        if (DEPTH) {
+            const float al = 1.0f - T;
+            depth_out[pid] = al > 1e-6f ? acc[CH] / al : 0.0f;
+        }
+    }
+    if (work) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) last = max(last, __shfl_xor(last, o, kWave));
+        if (lane == 0) atomicMax(&work[tile], last);  // cleared with the order
+    }
+}
+
+// Frames up to this many tiles take k_raster_fwd_split, whose four waves per
+// quadrant a larger frame has no room for.  Against k_raster_fwd (us, 10k
+// Gaussians in a blob / 30k in a box / 60k on shells): 256 tiles 105 / 62 / 72
+// -> 85 / 54 / 63, 520 tiles 92 / 52 / 66 -> 75 / 49 / 61, 690 tiles 84 / 48 /
+// 58 -> 69 / 58 / 67, 1024 tiles 73 / 42 / 49 -> 59 / 70 / 94.
+constexpr int kSplitTiles = 512;
 
 // Per-pixel state of the back-to-front replay.
 //
@@ -1019,7 +1311,7 @@ __global__ __launch_bounds__(kThreads, bwd_min_waves(CH)) void k_raster_bwd(
             for (int k = 0; k < BB * NV4 / kWave; ++k)
                 p[k * kWave + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
-        const int cnt = build_list<NLW, true>(s_mask[wave], s_list[wave], lane, BB * 16);
+        const int cnt = build_list<NLW, true>(s_mask[wave], s_list[wave], lane, 16, BB);
         const int lim = 16 * max(0, min(st.last - b * BB, BB));
         if (batch_plain)
             bwd_walk<CH, true>(s_list[wave], cnt, lim, s_r0, s_r1, s_f, s_part[wave], pxf, pyf,
@@ -1149,8 +1441,6 @@ struct BwdShape {
     static constexpr int NO = CHP + 8;  // row stride of a bucket's gradients in LDS
 };
 
-template <int V>
-using Int = std::integral_constant<int, V>;
 
 // The gradient outputs: the geometric ones in one record per Gaussian (xy,
 // stride floats) or in three arrays; feat + feat_stride * id + c is channel c
@@ -1247,13 +1537,6 @@ struct BwdLds {
     float* out;   // a bucket's gradients, rows of NO (6 geometric, then channels)
     int* id;      // its Gaussians (-1: none)
 };
-
-// The lane's index from the execution hardware, opaque to the compiler.
-__device__ __forceinline__ int lane_again() {
-    uint32_t z = 0;
-    asm volatile("" : "+s"(z));
-    return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, z));
-}
 
 // One bucket: the entries b0 .. b0 + 15 of the buffer, of which those below cnt
 // are real.  PLAIN: every one passed plain_gaussian and the quadrant's
@@ -2043,7 +2326,7 @@ __global__ __launch_bounds__(kThreads, 3) void k_raster_fwd_mx(
         const bool batch_plain = (pl.x & pl.y & pl.z & pl.w) != 0u;
         const bool batch_finite = (fi.x & fi.y & fi.z & fi.w) != 0u;
         if (alive == 0ull) continue;
-        const int cnt = build_list<NLW, false>(s_mask[wave], s_list[wave], lane, BB * 16);
+        const int cnt = build_list<NLW, false>(s_mask[wave], s_list[wave], lane, 16, BB);
         int last_off = -1;
         if (batch_finite) {
             if (batch_plain)
@@ -2195,14 +2478,31 @@ void launch_fwd(dim3 grid, hipStream_t st, bool depth, const float2* xy, const f
             hipLaunchKernelGGL((k_raster_fwd_mx<false>), grid, dim3(kThreads), 0, st, xy, co,
                                feat, C, c0, nc, depths, ids, ranges, n, n_ids, bg, W, H, tiles_x,
                                out, fT, ncon, dout, aout, order, work);
-    } else if (depth) {
-        hipLaunchKernelGGL((k_raster_fwd<CH, true>), grid, dim3(kThreads), 0, st, xy, co, feat, C,
-                           c0, nc, depths, ids, ranges, n, n_ids, bg, W, H, tiles_x, out, fT,
-                           ncon, dout, aout, order, work);
-    } else {
-        hipLaunchKernelGGL((k_raster_fwd<CH, false>), grid, dim3(kThreads), 0, st, xy, co, feat, C,
-                           c0, nc, depths, ids, ranges, n, n_ids, bg, W, H, tiles_x, out, fT,
-                           ncon, dout, aout, order, work);
+        return;
+    }
+    if constexpr (CH <= 4) {
+        if ((int)grid.x <= kSplitTiles && C <= 4) {
+            const dim3 wgs(32u * ((grid.x + 7u) / 8u));
+            if (depth)
+                hipLaunchKernelGGL((k_raster_fwd_split<CH, true>), wgs, dim3(kThreads), 0, st, xy,
+                                   co, feat, C, nc, depths, ids, ranges, n, n_ids, bg, W, H,
+                                   tiles_x, (int)grid.x, out, fT, ncon, dout, aout, order, work);
+            else
+                hipLaunchKernelGGL((k_raster_fwd_split<CH, false>), wgs, dim3(kThreads), 0, st,
+                                   xy, co, feat, C, nc, depths, ids, ranges, n, n_ids, bg, W, H,
+                                   tiles_x, (int)grid.x, out, fT, ncon, dout, aout, order, work);
+            return;
+        }
+    }
+    if constexpr (CH < 32) {
+        if (depth)
+            hipLaunchKernelGGL((k_raster_fwd<CH, true>), grid, dim3(kThreads), 0, st, xy, co,
+                               feat, C, c0, nc, depths, ids, ranges, n, n_ids, bg, W, H, tiles_x,
+                               out, fT, ncon, dout, aout, order, work);
+        else
+            hipLaunchKernelGGL((k_raster_fwd<CH, false>), grid, dim3(kThreads), 0, st, xy, co,
+                               feat, C, c0, nc, depths, ids, ranges, n, n_ids, bg, W, H, tiles_x,
+                               out, fT, ncon, dout, aout, order, work);
     }
 }
 

@@ -214,6 +214,9 @@ __device__ __forceinline__ void tile_order_band(int band, const int2* __restrict
             const int rank = (int)(s_cnt[(bk[k] * kBandItems + k) * (THREADS / kWave) + wave] +
                                    rk[k]) + (r0 - lo);
             order[BWD ? kOrderBands * rank + band : lo + rank] = t;
+            // the tile's bound (the words before the order), which a forward
+            // of one workgroup per quadrant raises with atomics
+            if (!BWD) order[t - tiles] = 0;
         }
         __syncthreads();
         // counters back to zero for the next round

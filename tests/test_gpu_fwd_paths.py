@@ -1,0 +1,62 @@
+"""The forward rasterizer's routes by frame size: frames of a few hundred tiles
+(one workgroup per quadrant), middle ones (the XCDs take the bands' lists in
+turns) and large ones.  One scene is drawn into canvases of every route; its
+pixels must be the same bits, whatever the canvas."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _frame(W, H, C, depth, plain, n=900):
+    """(outputs cropped to the scene's 96 x 80 pixels, tile bounds) of a W x H canvas."""
+    import torch
+
+    from mlx3d_amd.splatting.rasterize import raster_forward, tile_order_buffer
+    from mlx3d_amd.splatting.tiles import bin_gaussians
+
+    rng = np.random.default_rng(17 + C)
+    cu = lambda a: torch.from_numpy(np.ascontiguousarray(a, np.float32)).cuda()  # noqa: E731
+    xy = rng.uniform([-4, -4], [100, 84], (n, 2))
+    a = rng.uniform(0.02, 0.5, n)
+    c = rng.uniform(0.02, 0.5, n)
+    b = rng.uniform(-0.7, 0.7, n) * np.sqrt(a * c)
+    op = rng.uniform(0.0, 1.2, n)
+    op[::40] = 0.0
+    if not plain:  # a singular conic, a huge opacity and an infinite channel
+        b[5] = np.sqrt(a[5] * c[5])
+        op[9] = 1e31
+    feats = rng.standard_normal((n, C))
+    if not plain:
+        feats[11, 0] = np.inf
+    co = cu(np.stack([a, b, c, op], 1))
+    z = cu(rng.uniform(1, 9, n))
+    ids, ranges, _, _ = bin_gaussians(cu(xy), cu(np.full(n, 24.0)), z, W, H)
+    order = tile_order_buffer(W, H, co.device)
+    order.fill_(0)
+    bg = cu(rng.standard_normal(C))
+    out = raster_forward(cu(xy), co, cu(feats), ids, ranges, bg, W, H,
+                         depths=z if depth else None, tile_order=order)
+    tx, ty = (W + 15) // 16, (H + 15) // 16
+    bounds = order[:tx * ty].view(ty, tx)[:5, :6].cpu().numpy()
+    crop = [None if t is None else t[:80, :96].contiguous().cpu().numpy() for t in out]
+    return crop, bounds
+
+
+@pytest.mark.parametrize("C,depth,plain", [(1, False, True), (2, True, True), (3, False, True),
+                                           (3, True, True), (4, True, True), (3, True, False),
+                                           (5, False, True), (16, True, True)])
+def test_frame_sizes_agree(C, depth, plain):
+    # 30, 396 | 525, 3600 | 6500 tiles
+    base, bounds = _frame(96, 80, C, depth, plain)
+    n_contrib = base[2]
+    tiles = n_contrib.reshape(5, 16, 6, 16).max(axis=(1, 3))
+    np.testing.assert_array_equal(bounds, tiles)
+    assert int(n_contrib.max()) > 48  # several chunks of a workgroup's list
+    for W, H in ((352, 288), (400, 336), (1280, 720), (1600, 1040)):
+        got, b = _frame(W, H, C, depth, plain)
+        np.testing.assert_array_equal(b, bounds)
+        for name, x, y in zip(("out", "final_T", "n_contrib", "depth", "alpha"), base, got):
+            if x is not None:
+                np.testing.assert_array_equal(x, y, err_msg=f"{name} {W}x{H}")
