@@ -431,8 +431,8 @@ __device__ __forceinline__ float comp4(const float4& v, int e) {
 // and padded channels (12 registers) kept the LDS busy for 82 of the 91
 // million cycles in which a CU had work (1M Gaussians, 1080p), so a record
 // holds nothing the loop can do without: 177 -> 166 us there, 188 -> 179 us
-// with 3M.  A wave alone on its SIMD gains nothing from it (a crowded tile of
-// Gaussians in a blob at 690 tiles: 169 -> 178 us with 60k).
+// with 3M.  A wave alone on its SIMD gains nothing from it (a blob of 60k
+// Gaussians at 690 tiles, bound by one crowded tile: 169 -> 178 us).
 template <int NV>
 struct FwdRec {
     static constexpr int EX = NV > 2 ? NV - 2 : 0;
