@@ -88,3 +88,48 @@ def test_wide_backward_non_finite(C):
         assert fin.any()
         e = float(np.abs(a[fin] - b[fin]).max() / (np.abs(b[fin]).max() + 1e-30))
         assert e < 1e-4, k
+
+
+@pytest.mark.parametrize("plain", [True, False])
+@pytest.mark.parametrize("by_pixel", [True, False])
+@pytest.mark.parametrize("C", [5, 9, 17])
+def test_wide_backward_behind_opaque(C, by_pixel, plain):
+    """The colour behind an opaque entry, which dL/dalpha divides by 1 - alpha =
+    0.01: stacks of three Gaussians, each on one pixel alone (the middle one at the
+    0.99 clamp, a dim one behind it), against 64 bits, in list orders that put a
+    stack's entries side by side and a layer apart."""
+    from mlx3d_amd.splatting.rasterize import (pack_conic_opacity, raster_backward_geometry,
+                                               raster_forward)
+
+    W = H = 32
+    P, L = W * H, 3
+    rng = np.random.default_rng(C)
+    layer, pixel = np.divmod(np.arange(L * P), P)
+    m2 = np.stack([pixel % W + 0.5, pixel // W + 0.5], 1).astype(np.float32)
+    con = np.tile(np.array([30.0, 0.0, 30.0 if plain else 1e9], np.float32), (L * P, 1))
+    op = np.array([0.3, 1.0, 0.5], np.float32)[layer]
+    feats = rng.uniform(0.5, 1.0, (L * P, C)).astype(np.float32)
+    feats[layer == 2] *= np.float32(0.01)
+    g_img = rng.uniform(0.5, 1.0, (H, W, C)).astype(np.float32)
+    depths = 1.0 + (pixel * L + layer if by_pixel else layer * P + pixel).astype(np.float32)
+    ids, ranges, _, _ = bin_gaussians(cu(m2), cu(np.ones(L * P, np.float32)), cu(depths), W, H)
+    co = pack_conic_opacity(cu(con), cu(op))
+    _, fT, nc, _, _ = raster_forward(cu(m2), co, cu(feats), ids, ranges, None, W, H)
+    rec, _ = raster_backward_geometry(cu(m2), co, cu(feats), ids, ranges, None, W, H, fT, nc,
+                                      cu(g_img), None)
+    got = host(rec)[:, 5].astype(np.float64).reshape(L, P)  # dL/dopacity = dL/dalpha (G = 1)
+    # alpha is min(0.99, opacity) to the bit, so 64 bits start from the same values
+    alpha = np.minimum(np.float32(0.99), op).astype(np.float64).reshape(L, P)
+    cg = (feats.astype(np.float64).reshape(L, P, C) * g_img.reshape(1, P, C)).sum(-1)
+    T = np.cumprod(np.concatenate([np.ones((1, P)), 1.0 - alpha[:-1]]), 0)
+    term = alpha * T * cg
+    behind = term[::-1].cumsum(0)[::-1] - term
+    want = T * cg - behind / (1.0 - alpha)
+    scale = T * cg + behind / (1.0 - alpha)
+    # every term is positive.  T: three roundings of 1 - alpha and three products
+    # ahead, a reciprocal (1 ulp) and a product an entry back; c . g: C
+    # products and sums; alpha T, the sum behind, its quotient, the difference
+    # and h / opacity: at most (6 + 9 + C + 8) 2^-24 of the terms' size
+    e = np.abs(got - want) / scale
+    say(f"  C={C} by_pixel={by_pixel} plain={plain}: largest error {e.max(1)} of the terms")
+    assert e.max() < (23 + C) * 2.0 ** -24
