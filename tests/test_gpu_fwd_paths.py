@@ -60,3 +60,35 @@ def test_frame_sizes_agree(C, depth, plain):
         for name, x, y in zip(("out", "final_T", "n_contrib", "depth", "alpha"), base, got):
             if x is not None:
                 np.testing.assert_array_equal(x, y, err_msg=f"{name} {W}x{H}")
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 6, 255, 256, 257, 515])
+def test_needle_lists_match_oracle(n):
+    """Batches with an ill-conditioned conic, an opacity past the exp's range and
+    an infinite channel, in lists of every remainder of a round: the oracle's bits."""
+    from gpu_util import assert_bits, cu, host
+    from mlx3d_amd.splatting.rasterize import pack_conic_opacity, raster_forward
+    from mlx3d_amd.splatting.tiles import bin_gaussians
+    from oracle import oracle as O
+
+    W, H, C = 561, 369, 3  # a corner tile of 1 x 1 pixels
+    rng = np.random.default_rng(n)
+    xy = rng.uniform([W - 12, H - 12], [W + 2, H + 2], (n, 2)).astype(np.float32)
+    a, c = rng.uniform(0.01, 0.3, n), rng.uniform(0.01, 0.3, n)
+    con = np.stack([a, rng.uniform(-0.7, 0.7, n) * np.sqrt(a * c), c], 1).astype(np.float32)
+    op = rng.uniform(0.004, 0.1, n).astype(np.float32)
+    feats = rng.standard_normal((n, C)).astype(np.float32)
+    z = rng.uniform(1, 9, n).astype(np.float32)
+    k = n // 2
+    con[k], xy[k] = (1e3, 0.0, 1e-4), (W - 7.5, H - 40.0)
+    if n > 3:
+        op[0], feats[3, 1] = 1e31, np.inf
+    ids, ranges, _, _ = bin_gaussians(cu(xy), cu(np.full(n, 24.0, np.float32)), cu(z), W, H)
+    bg = rng.random(C, dtype=np.float32)
+    ref = O.raster_fwd(xy, con, op, feats, host(ids), host(ranges), W, H, bg=bg, depths=z)
+    out, fT, nc, depth, _ = raster_forward(cu(xy), pack_conic_opacity(cu(con), cu(op)), cu(feats),
+                                           ids, ranges, cu(bg), W, H, depths=cu(z))
+    assert ref["n_contrib"].max() >= min(n, 3) - 1
+    np.testing.assert_array_equal(host(nc), ref["n_contrib"])
+    for name, got in (("image", out), ("final_T", fT), ("depth", depth)):
+        assert_bits(host(got), ref[name], name)
