@@ -591,9 +591,22 @@ __device__ __forceinline__ void fwd_walk(const uint32_t* list, int cnt, const fl
     }
 }
 
-// Occupancy targets that the compiler meets without spilling: eight waves
-// per SIMD (<= 64 VGPRs) up to three channels, seven up to eight.
-constexpr int fwd_min_waves(int ch) { return ch <= 3 ? 8 : (ch <= 8 ? 7 : 4); }
+// Occupancy targets.  Up to four channels the kernel fits eight waves per SIMD
+// (<= 64 VGPRs) by itself; asking for eight or seven makes the compiler hold
+// back scalar registers too and move some through vector lanes in the staging
+// (60k on 690 tiles 171 us so, 169.5 without).
+constexpr int fwd_min_waves(int ch) { return ch <= 8 ? 6 : 4; }
+
+// The channel of value i in a block of nc of CH channels: groups of four that
+// lie inside the row, the last ones overlapping where nc < CH (their channels
+// are summed twice, with the same bits).  A group is then one load and no channel
+// takes a branch; with a branch per channel each was a load of its own (500k,
+// 720p: 16 channels 158 -> 130 us, 12 channels 144 -> 126, 3 channels 95 -> 91).
+// Up to four channels a block is whole.
+template <int CH>
+__device__ __forceinline__ int fwd_channel(int i, int nc) {
+    return CH <= 4 ? i : min(i & ~3, nc - 4) + (i & 3);
+}
 
 template <int CH, bool DEPTH>
 __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
@@ -660,8 +673,7 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
                 for (int i = 0; i < 4 * Rec::X4 + 2; ++i) v[i] = 0.0f;
                 const float* const f = feat + (int64_t)g * C + c0;
 #pragma unroll
-                for (int ch = 0; ch < CH; ++ch)
-                    if (nc >= CH || ch < nc) v[ch] = f[ch];
+                for (int i = 0; i < CH; ++i) v[i] = f[fwd_channel<CH>(i, nc)];
                 if (DEPTH) v[CH] = depths[g];
                 const float thr = alpha_floor_power(c.w);
                 float4* const r = reinterpret_cast<float4*>(s_rec + tid * RS);
@@ -702,8 +714,10 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
         const float T = p.T;
         float* o = out + pid * C + c0;
 #pragma unroll
-        for (int ch = 0; ch < CH; ++ch)
-            if (ch < nc) o[ch] = p.acc[ch] + T * (bg ? bg[c0 + ch] : 0.0f);
+        for (int i = 0; i < CH; ++i) {
+            const int ch = fwd_channel<CH>(i, nc);
+            o[ch] = p.acc[i] + T * (bg ? bg[c0 + ch] : 0.0f);
+        }
         if (c0 == 0) {
             final_T[pid] = T;
             n_contrib[pid] = last;
@@ -795,8 +809,7 @@ __global__ __launch_bounds__(kThreads) void k_raster_fwd_split(
                 c = co[g];
                 const float* const f = feat + (int64_t)g * C;
 #pragma unroll
-                for (int ch = 0; ch < CH; ++ch)
-                    if (nc >= CH || ch < nc) v[ch] = f[ch];
+                for (int ch = 0; ch < CH; ++ch) v[ch] = f[ch];  // CH == nc == C
                 if (DEPTH) v[CH] = depths[g];
                 keep = quadrant_reached(m.x, m.y, c, qx0, qy0);
                 thr = alpha_floor_power(c.w);

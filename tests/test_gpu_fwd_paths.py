@@ -92,3 +92,31 @@ def test_needle_lists_match_oracle(n):
     np.testing.assert_array_equal(host(nc), ref["n_contrib"])
     for name, got in (("image", out), ("final_T", fT), ("depth", depth)):
         assert_bits(host(got), ref[name], name)
+
+
+@pytest.mark.parametrize("C", [5, 6, 7, 9, 10, 11, 13, 14, 15, 16, 38, 41, 47])
+def test_channel_blocks_match_oracle(C):
+    """Every remainder of a block's groups of four channels (the last ones overlap),
+    the block's last channel infinite for one Gaussian: the oracle's bits."""
+    from gpu_util import assert_features, cu, host
+    from mlx3d_amd.splatting.rasterize import pack_conic_opacity, raster_forward
+    from mlx3d_amd.splatting.tiles import bin_gaussians
+    from oracle import oracle as O
+
+    W, H, n = 57, 41, 300
+    rng = np.random.default_rng(C)
+    xy = rng.uniform([-2, -2], [W + 2, H + 2], (n, 2)).astype(np.float32)
+    a, c = rng.uniform(0.02, 0.5, n), rng.uniform(0.02, 0.5, n)
+    con = np.stack([a, rng.uniform(-0.7, 0.7, n) * np.sqrt(a * c), c], 1).astype(np.float32)
+    op = rng.uniform(0.01, 0.6, n).astype(np.float32)
+    feats = rng.standard_normal((n, C)).astype(np.float32)
+    feats[17, C - 1] = np.inf
+    ids, ranges, _, _ = bin_gaussians(cu(xy), cu(np.full(n, 16.0, np.float32)),
+                                      cu(rng.uniform(1, 9, n).astype(np.float32)), W, H)
+    bg = rng.random(C, dtype=np.float32)
+    ref = O.raster_fwd(xy, con, op, feats, host(ids), host(ranges), W, H, bg=bg)
+    out, _, nc, _, _ = raster_forward(cu(xy), pack_conic_opacity(cu(con), cu(op)), cu(feats),
+                                      ids, ranges, cu(bg), W, H)
+    assert np.isinf(ref["image"][..., C - 1]).any()
+    np.testing.assert_array_equal(host(nc), ref["n_contrib"])
+    assert_features(host(out), ref["image"])
