@@ -430,29 +430,29 @@ __device__ __forceinline__ float comp4(const float4& v, int e) {
 // per register it fills, broadcast or not: a separate log-alpha bound, depth
 // and padded channels (12 registers) kept the LDS busy for 82 of the 91
 // million cycles in which a CU had work (1M Gaussians, 1080p), so a record
-// holds nothing the loop can do without: 177 -> 166 us there, 188 -> 179 us
-// with 3M.  A wave alone on its SIMD gains nothing from it (a blob of 60k
-// Gaussians at 690 tiles, bound by one crowded tile: 169 -> 178 us).
+// holds nothing the loop can do without.  Its 16-byte pieces lie in arrays of
+// their own, which a walk addresses by one offset of 16 x the staged index
+// (whole records of 32 to 96 bytes took up to six more registers and 0.5 to
+// 2 % longer, 16 channels 1 % less).
+constexpr int kRecords = kThreads + 1;  // the last is the walk lists' padding
 template <int NV>
 struct FwdRec {
     static constexpr int EX = NV > 2 ? NV - 2 : 0;
     static constexpr int X4 = (EX + 3) / 4;
-    static constexpr int kStride = 8 + 4 * X4;  // floats
+    static constexpr int kPieces = 2 + X4;
     float4 r0, r1;
     float x[4 * X4 + 1];
     __device__ __forceinline__ float value(int i) const {
         return i == 0 ? r0.w : (i == 1 ? r1.w : x[i - 2]);
     }
-    // the byte offset is a multiple of the stride
-    __device__ __forceinline__ void load(const float* base, uint32_t off) {
-        const char* p = reinterpret_cast<const char*>(base) + off;
-        r0 = *reinterpret_cast<const float4*>(p);
-        r1 = *reinterpret_cast<const float4*>(p + 16);
+    __device__ __forceinline__ void load(const float4* base, uint32_t off) {
+        r0 = rec_at(base, off);
+        r1 = rec_at(base + kRecords, off);
     }
-    __device__ __forceinline__ void load_values(const float* base, uint32_t off) {
-        const char* p = reinterpret_cast<const char*>(base) + off + 32;
+    __device__ __forceinline__ void load_values(const float4* base, uint32_t off) {
+        const float4* const p = &rec_at(base + 2 * kRecords, off);
         if constexpr (EX == 1) {
-            x[0] = *reinterpret_cast<const float*>(p);
+            x[0] = p->x;
         } else if constexpr (EX == 2) {
             const float2 v = *reinterpret_cast<const float2*>(p);
             x[0] = v.x;
@@ -460,7 +460,7 @@ struct FwdRec {
         } else if constexpr (EX > 2) {
 #pragma unroll
             for (int k = 0; k < X4; ++k) {
-                const float4 v = reinterpret_cast<const float4*>(p)[k];
+                const float4 v = p[k * kRecords];
                 x[4 * k] = v.x;
                 x[4 * k + 1] = v.y;
                 x[4 * k + 2] = v.z;
@@ -540,7 +540,7 @@ __device__ __forceinline__ void fwd_pair(const FwdRec<NV>& g, int off, FwdPixel<
 // The wave stops once its 64 pixels have terminated.  last_off gets the
 // offset of each pixel's last composited Gaussian of this batch.
 template <int NV, bool PLAIN>
-__device__ __forceinline__ void fwd_walk(const uint32_t* list, int cnt, const float* rec,
+__device__ __forceinline__ void fwd_walk(const uint32_t* list, int cnt, const float4* rec,
                                          FwdPixel<NV>& px, uint64_t& alive) {
     using Rec = FwdRec<NV>;
     // more values are read just before their pair (registers)
@@ -618,9 +618,8 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
     const int* __restrict__ order, int* __restrict__ work) {
     constexpr int NV = CH + (DEPTH ? 1 : 0);
     using Rec = FwdRec<NV>;
-    constexpr int RS = Rec::kStride;
     // record kThreads is the lists' padding: opacity zero, which no pixel takes
-    __shared__ __align__(16) float s_rec[(kThreads + 1) * RS];
+    __shared__ float4 s_rec[Rec::kPieces * kRecords];
     __shared__ uint64_t s_mask[kWaves][kWaves];  // [quadrant][loader wave]
     __shared__ uint32_t s_list[kWaves][kThreads + 8];  // walk lists (+ look-ahead room)
     // one word per wave, written before a barrier and read by every thread
@@ -651,7 +650,8 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
     int last = 0;
     uint64_t alive = __ballot(inside);  // the wave's pixels still compositing
     // the padding record (written before the first barrier)
-    if (tid < RS) s_rec[kThreads * RS + tid] = 0.0f;
+    if (tid < Rec::kPieces)
+        s_rec[tid * kRecords + kThreads] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 
     for (int base = 0; base < num; base += kThreads) {
         const int lane = lane_again(), tid = wave * kWave + lane;
@@ -676,13 +676,13 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
                 for (int i = 0; i < CH; ++i) v[i] = f[fwd_channel<CH>(i, nc)];
                 if (DEPTH) v[CH] = depths[g];
                 const float thr = alpha_floor_power(c.w);
-                float4* const r = reinterpret_cast<float4*>(s_rec + tid * RS);
+                float4* const r = s_rec + tid;
                 r[0] = make_float4(m.x, m.y, c.w, v[0]);
-                r[1] = make_float4(-0.5f * c.x, -c.y, -0.5f * c.z, v[1]);
+                r[kRecords] = make_float4(-0.5f * c.x, -c.y, -0.5f * c.z, v[1]);
 #pragma unroll
                 for (int i = 0; i < Rec::X4; ++i)
-                    r[2 + i] = make_float4(v[2 + 4 * i], v[3 + 4 * i], v[4 + 4 * i],
-                                           v[5 + 4 * i]);
+                    r[(2 + i) * kRecords] = make_float4(v[2 + 4 * i], v[3 + 4 * i],
+                                                        v[4 + 4 * i], v[5 + 4 * i]);
                 qm = quadrant_mask(m.x, m.y, c, px0, py0);
                 plain = plain_gaussian<0>(m.x, m.y, c, thr, nullptr);
 #pragma unroll
@@ -701,13 +701,13 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
         const bool batch_plain = (pl.x & pl.y & pl.z & pl.w) != 0u;
         if (alive == 0ull) continue;
         const int cnt =
-            build_list<kWaves, false, 4>(s_mask[wave], s_list[wave], lane, 4 * RS, kThreads);
+            build_list<kWaves, false, 4>(s_mask[wave], s_list[wave], lane, 16, kThreads);
         p.last_off = -1;
         if (batch_plain)
             fwd_walk<NV, true>(s_list[wave], cnt, s_rec, p, alive);
         else
             fwd_walk<NV, false>(s_list[wave], cnt, s_rec, p, alive);
-        if (p.last_off >= 0) last = base + (int)((uint32_t)p.last_off / (4u * RS)) + 1;
+        if (p.last_off >= 0) last = base + (p.last_off >> 4) + 1;
     }
     if (inside) {
         const int64_t pid = (int64_t)py * W + px;
