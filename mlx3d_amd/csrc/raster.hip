@@ -734,8 +734,8 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
 // The forward of small frames.  One wave composites a quadrant's list serially
 // in k_raster_fwd, about 45 instructions an entry, and a wave alone on its
 // SIMD issues one every six cycles: the tile with the longest list bounds the
-// launch (1889 entries: 106 us of a 256 x 256 view, 86 us here).  Only the chain through
-// T is serial, so here a workgroup has one quadrant: three waves evaluate
+// launch (2221 entries of a 256 x 256 view: 106 us, 87 us here).  Only the chain
+// through T is serial, so here a workgroup has one quadrant: three waves evaluate
 // alphas, 16 entries of a chunk of 48 each, into LDS (zero where the pixel
 // does not take the entry), while wave 0 composites the chunk before.  The
 // arithmetic of a pair is fwd_pair's, so every output has its bits: an alpha
@@ -934,12 +934,17 @@ __global__ __launch_bounds__(kThreads) void k_raster_fwd_split(
     }
 }
 
-// Frames up to this many tiles take k_raster_fwd_split, whose four waves per
-// quadrant a larger frame has no room for.  Against k_raster_fwd (us, 10k
-// Gaussians in a blob / 30k in a box / 60k on shells): 256 tiles 105 / 62 / 72
-// -> 85 / 54 / 63, 520 tiles 92 / 52 / 66 -> 75 / 49 / 61, 690 tiles 84 / 48 /
-// 58 -> 69 / 58 / 67, 1024 tiles 73 / 42 / 49 -> 59 / 70 / 94.
-constexpr int kSplitTiles = 512;
+// Frames up to this many tiles take k_raster_fwd_split: all of its four workgroups
+// per tile then have a place at once on 256 compute units, whose LDS holds four
+// each (37 KB up to four values), or three (41 KB).  In two rounds it loses
+// wherever the work is spread over the frame, and splitting only as many of the
+// longest lists as leave every workgroup a place still lost up to 25 % there.
+// k_raster_fwd -> k_raster_fwd_split, us, for 10k in a blob, 300k in a box, 1M
+// on shells, 400k with heavy tails: 110 tiles 153 -> 121, 268 -> 184, 169 -> 143,
+// 39 -> 35; 169 tiles 128 -> 103, 176 -> 130, 138 -> 125, 33 -> 34; 256 tiles
+// 106 -> 87, 123 -> 97, 114 -> 102, 31 -> 31; 342 tiles 101 -> 83, 113 -> 96,
+// 110 -> 136, 30 -> 45; 510 tiles 104 -> 85, 129 -> 103, 113 -> 145, 32 -> 53.
+constexpr int split_tiles(int values) { return values <= 4 ? 256 : 192; }
 
 // Per-pixel state of the back-to-front replay.
 //
@@ -2515,7 +2520,7 @@ void launch_fwd(dim3 grid, hipStream_t st, bool depth, const float2* xy, const f
         return;
     }
     if constexpr (CH <= 4) {
-        if ((int)grid.x <= kSplitTiles && C <= 4) {
+        if ((int)grid.x <= split_tiles(CH + (depth ? 1 : 0)) && C <= 4) {
             const dim3 wgs(32u * ((grid.x + 7u) / 8u));
             if (depth)
                 hipLaunchKernelGGL((k_raster_fwd_split<CH, true>), wgs, dim3(kThreads), 0, st, xy,

@@ -48,13 +48,14 @@ def _frame(W, H, C, depth, plain, n=900):
                                            (3, True, True), (4, True, True), (3, True, False),
                                            (5, False, True), (16, True, True)])
 def test_frame_sizes_agree(C, depth, plain):
-    # 30, 396 | 525, 3600 | 6500 tiles
+    # 30, 192 | 208, 256 | 272, 396, 525, 3600, 6500 tiles
     base, bounds = _frame(96, 80, C, depth, plain)
     n_contrib = base[2]
     tiles = n_contrib.reshape(5, 16, 6, 16).max(axis=(1, 3))
     np.testing.assert_array_equal(bounds, tiles)
     assert int(n_contrib.max()) > 48  # several chunks of a workgroup's list
-    for W, H in ((352, 288), (400, 336), (1280, 720), (1600, 1040)):
+    for W, H in ((192, 256), (208, 256), (256, 256), (272, 256), (352, 288), (400, 336),
+                 (1280, 720), (1600, 1040)):
         got, b = _frame(W, H, C, depth, plain)
         np.testing.assert_array_equal(b, bounds)
         for name, x, y in zip(("out", "final_T", "n_contrib", "depth", "alpha"), base, got):
