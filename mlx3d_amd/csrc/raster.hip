@@ -330,20 +330,18 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
 // balanced as well but doubled the rasterizers' HBM traffic (1.05 GB per
 // C3 backward instead of 0.47: neighbouring tiles on different XCDs).
 // by_block: order is indexed by workgroup (the backward's layout, -1 = no
-// tile), else by xcd_remap position.  The forward does not know a tile's work
-// beforehand, and a scene's crowded region fills a few bands: the busiest
-// XCD had 1.4 to 1.5 times the mean work at 3600 to 4096 tiles.  Up to
-// kDealTiles tiles its workgroups therefore take the bands' lists in turns
-// of eight ranks, each XCD an eighth of every band: 106 -> 94 us (300k
-// through a fisheye, 4096 tiles), 267 -> 239 us (32 channels, 500k, 3600
-// tiles), 82 -> 80 us (200k, 2040 tiles).  With 8160 tiles of 1M and 3M
-// Gaussians the bands' work is even (1.06, 1.04) and the lost locality
-// shows, 177 -> 180 and 188 -> 195 us, so larger frames keep whole bands.
-constexpr uint32_t kDealTiles = 6144;
+// tile).  The forward does not know a tile's work beforehand, and a scene's
+// crowded region fills a few of its bands: the busiest XCD's lists hold 1.1 to
+// 3.5 times the mean.  Its workgroups therefore take the bands' lists in turns of
+// eight ranks, each XCD an eighth of every band.  Whole bands -> turns, us, at
+// 1200 / 3600 / 8160 / 32400 tiles: a blob (300k) 232 -> 230, 176 -> 161, 197 ->
+// 137, 512 -> 279; a box (300k) 82 -> 81, 79 -> 80, 103 -> 97; heavy tails (400k;
+// 1M at 32400) 38 -> 37, 69 -> 67, 126 -> 120, 432 -> 418; shells (1M), where
+// neighbouring tiles share the most, 85 -> 89, 104 -> 106, 178 -> 170, 457 -> 457;
+// 32 channels, 1M in a box at 8160 tiles, 451 -> 381.
 __device__ __forceinline__ int tile_at(const int* order, uint32_t b, uint32_t nb, bool by_block) {
     if (!order) return (int)xcd_remap(b, nb);
     if (by_block) return order[b];
-    if (nb > kDealTiles) return order[xcd_remap(b, nb)];
     const uint32_t q = nb / 8u, r = nb % 8u, i = b / 8u, x = b % 8u;
     const uint32_t band = i < q ? (x + (i >> 3)) & 7u : x;
     return order[band * q + min(band, r) + i];
