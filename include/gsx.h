@@ -425,6 +425,24 @@ int gsx_raster_bwd_geometry(int64_t n, int32_t C, const float* means2d,
                             float* g_features, int32_t grad_stride,
                             int32_t* tile_order, void* stream);
 
+/* The same for C of 5 to 32 with rows the caller spaces: the features'
+ * gradient of Gaussian i lies at g_features + i * feature_stride (>= C floats),
+ * or, with g_features NULL, behind its geometric six in the record (grad_stride
+ * >= 6 + C).  The atomics of a Gaussian cost one unit per 64-byte line they
+ * touch, so rows that do not straddle lines (16 floats, a record of 16 up to ten
+ * channels) serve Gaussians that reach many tiles.  Words past a row's C
+ * channels are cleared. */
+int gsx_raster_bwd_rows(int64_t n, int32_t C, const float* means2d,
+                        const float* conic_opacity, const float* features,
+                        const int32_t* sorted_ids, int64_t num_ids,
+                        const int32_t* tile_ranges, const float* background,
+                        int32_t width, int32_t height, const float* final_T,
+                        const int32_t* n_contrib, const float* grad_out,
+                        const float* grad_final_T, float* g_geometry,
+                        int32_t grad_stride, float* g_features,
+                        int32_t feature_stride, int32_t* tile_order,
+                        void* stream);
+
 int gsx_split_raster_grads(int64_t n, const float* record, int32_t grad_stride,
                            float* g_means2d, float* g_conics,
                            float* g_opacities, void* stream);

@@ -150,6 +150,8 @@ SIGNATURES = {
                                       _P, _P, _P, _P, _P, _P, _P, _I32, _P, _P]),
     "gsx_raster_bwd_geometry": (ctypes.c_int, [_I64, _I32, _P, _P, _P, _P, _I64, _P, _P, _I32,
                                                _I32, _P, _P, _P, _P, _P, _P, _I32, _P, _P]),
+    "gsx_raster_bwd_rows": (ctypes.c_int, [_I64, _I32, _P, _P, _P, _P, _I64, _P, _P, _I32, _I32,
+                                           _P, _P, _P, _P, _P, _I32, _P, _I32, _P, _P]),
     "gsx_split_raster_grads": (ctypes.c_int, [_I64, _P, _I32, _P, _P, _P, _P]),
     "gsx_photometric_workspace_bytes": (_I64, [_I32, _I32, _I32]),
     "gsx_photometric_fwd": (ctypes.c_int, [_I32, _I32, _I32, _P, _P, _I32, _F, _F, _P, _I64, _P,

@@ -1470,6 +1470,15 @@ struct BwdShape {
 // The gradient outputs: the geometric ones in one record per Gaussian (xy,
 // stride floats) or in three arrays; feat + feat_stride * id + c is channel c
 // of the block, in the record or in an array of its own.
+//
+// Where Gaussians reach many tiles the atomics' lines bind (bwd_send).  Rows of
+// C floats straddle 64-byte lines unless C is a multiple of 16, so callers then
+// ask for rows of 16, or up to ten channels for a record of 16 that holds all,
+// and copy the features out.  Rows of C -> whole lines with the copy, us: 300k with
+// heavy tails at 960 x 540 (7 tiles each) 228 -> 159 (5 channels), 273 -> 214
+// (12); 500k on shells at 1080p (10) 466 -> 437, 541 -> 502; 60k at 641 x 479
+// (8; 0.5M duplicates) 121 -> 120, 142 -> 134; 500k in a box at 720p (3) 202 ->
+// 203, 247 -> 246.
 struct BwdOut {
     float* xy;
     float* conic;
@@ -1847,7 +1856,7 @@ __global__ __launch_bounds__(kWave, bwd_wide_waves(CHP)) void k_raster_bwd_wide(
     const float* __restrict__ final_T, const int* __restrict__ n_contrib,
     const float* __restrict__ grad_out, const float* __restrict__ grad_T,
     float* __restrict__ g_xy, float* __restrict__ g_conic, float* __restrict__ g_feat,
-    float* __restrict__ g_opac, int gstride, const int* __restrict__ order) {
+    float* __restrict__ g_opac, int gstride, int fstride, const int* __restrict__ order) {
     using S = BwdShape<CHP>;
     constexpr int GS = CHP < 16 ? CHP : 16;
     // wide blocks' cotangents pass through the records' space, 16 channels of
@@ -1957,13 +1966,13 @@ __global__ __launch_bounds__(kWave, bwd_wide_waves(CHP)) void k_raster_bwd_wide(
     O.xy = g_xy;
     O.conic = g_conic;
     O.opac = g_opac;
-    O.feat = g_feat ? g_feat + c0 : g_xy + 6 + c0;
-    O.feat_stride = g_feat ? C : gstride;
+    O.feat = g_feat + c0;
+    O.feat_stride = fstride;
     O.stride = gstride;
     O.nc = nc;
     O.C = C;
     // a block's channels follow the geometric gradients in its record
-    O.whole = O.record && !g_feat && c0 == 0;
+    O.whole = O.record && g_feat == g_xy + 6 && c0 == 0;
     const int comps = O.whole ? 6 + nc : nc;
     O.per = kWave / comps;
     O.mul = 65536 / comps + 1;
@@ -2548,13 +2557,13 @@ void launch_bwd(int slots, hipStream_t st, const float2* xy, const float4* co, c
                 int C, int c0, int nc, const int* ids, const int2* ranges, int64_t n,
                 int64_t n_ids, const float* bg, int W, int H, int tiles_x, const float* fT,
                 const int* ncon, const float* gout, const float* gT, float* gxy, float* gcon,
-                float* gfeat, float* gop, int gstride, const int* order) {
+                float* gfeat, float* gop, int gstride, int fstride, const int* order) {
     if constexpr (CH > 4)
         // four quadrant workgroups per tile slot, slots in groups of eight (XCDs)
         hipLaunchKernelGGL((k_raster_bwd_wide<CH>), dim3(32u * (((unsigned)slots + 7u) / 8u)),
                            dim3(kWave), 0, st, xy, co, feat, C, c0, nc, ids, ranges, n, n_ids, bg,
-                           W, H, tiles_x, slots, fT, ncon, gout, gT, gxy, gcon, gfeat, gop,
-                           gstride, order);
+                           W, H, tiles_x, slots, fT, ncon, gout, gT, gxy, gcon,
+                           gfeat ? gfeat : gxy + 6, gop, gstride, fstride, order);
     else
         hipLaunchKernelGGL((k_raster_bwd<CH>), dim3((unsigned)slots), dim3(kThreads), 0, st, xy,
                            co, feat, C, c0, nc, ids, ranges, n, n_ids, bg, W, H, tiles_x, fT,
@@ -2564,14 +2573,16 @@ void launch_bwd(int slots, hipStream_t st, const float2* xy, const float4* co, c
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 inline bool aligned8(const void* p) { return ((uintptr_t)p & 7u) == 0; }
 
-// The backward into the outputs the two entry points accept.
+// The backward into the outputs that the entry points accept; feature_stride:
+// floats from one Gaussian's feature gradient to the next.
 int raster_bwd(int64_t n, int32_t C, const float* means2d, const float* conic_opacity,
                    const float* features, const int32_t* sorted_ids, int64_t num_ids,
                    const int32_t* tile_ranges,
                    const float* background, int32_t width, int32_t height, const float* final_T,
                    const int32_t* n_contrib, const float* grad_out, const float* grad_final_T,
                    float* g_means2d, float* g_conics, float* g_features, float* g_opacities,
-                   int32_t grad_stride, int32_t* tile_order, void* stream) {
+                   int32_t grad_stride, int32_t feature_stride, int32_t* tile_order,
+                   void* stream) {
     if (n < 0 || num_ids < 0 || C <= 0 || width <= 0 || height <= 0) return GSX_ERR_INVALID;
     if (!tile_ranges || !final_T || !n_contrib || !grad_out) return GSX_ERR_INVALID;
     const bool rec = grad_stride > 0;
@@ -2598,7 +2609,7 @@ int raster_bwd(int64_t n, int32_t C, const float* means2d, const float* conic_op
             z.p[0] = g_means2d;
             z.n[0] = (int64_t)grad_stride * n;
             z.p[2] = g_features;
-            z.n[2] = g_features ? (int64_t)C * n : 0;
+            z.n[2] = g_features ? (int64_t)feature_stride * n : 0;
         } else {
             z.p[0] = g_means2d;
             z.n[0] = 2 * n;
@@ -2626,7 +2637,8 @@ int raster_bwd(int64_t n, int32_t C, const float* means2d, const float* conic_op
         launch_bwd<V>(slots, st, (const float2*)means2d, (const float4*)conic_opacity, features, \
                       C, c0, nc, sorted_ids, (const int2*)tile_ranges, n, num_ids, background,   \
                       width, height, tiles_x, final_T, n_contrib, grad_out, grad_final_T,        \
-                      g_means2d, g_conics, g_features, g_opacities, grad_stride, order);         \
+                      g_means2d, g_conics, g_features, g_opacities, grad_stride, feature_stride, \
+                      order);                                                                    \
         break;
             GSX_BWD_CASE(1)
             GSX_BWD_CASE(2)
@@ -2725,8 +2737,8 @@ int gsx_raster_bwd(int64_t n, int32_t C, const float* means2d, const float* coni
         return GSX_ERR_INVALID;
     return raster_bwd(n, C, means2d, conic_opacity, features, sorted_ids, num_ids, tile_ranges,
                       background, width, height, final_T, n_contrib, grad_out, grad_final_T,
-                      g_means2d, g_conics, g_features, g_opacities, grad_stride, tile_order,
-                      stream);
+                      g_means2d, g_conics, g_features, g_opacities, grad_stride,
+                      rec ? grad_stride : C, tile_order, stream);
 }
 
 int gsx_raster_bwd_geometry(int64_t n, int32_t C, const float* means2d, const float* conic_opacity,
@@ -2740,7 +2752,25 @@ int gsx_raster_bwd_geometry(int64_t n, int32_t C, const float* means2d, const fl
     if (n > 0 && !g_features) return GSX_ERR_INVALID;
     return raster_bwd(n, C, means2d, conic_opacity, features, sorted_ids, num_ids, tile_ranges,
                       background, width, height, final_T, n_contrib, grad_out, grad_final_T,
-                      g_geometry, nullptr, g_features, nullptr, grad_stride, tile_order, stream);
+                      g_geometry, nullptr, g_features, nullptr, grad_stride, C, tile_order, stream);
+}
+
+int gsx_raster_bwd_rows(int64_t n, int32_t C, const float* means2d, const float* conic_opacity,
+                        const float* features, const int32_t* sorted_ids, int64_t num_ids,
+                        const int32_t* tile_ranges, const float* background, int32_t width,
+                        int32_t height, const float* final_T, const int32_t* n_contrib,
+                        const float* grad_out, const float* grad_final_T, float* g_geometry,
+                        int32_t grad_stride, float* g_features, int32_t feature_stride,
+                        int32_t* tile_order, void* stream) {
+    if (C < 5 || C > kMaxChunk || grad_stride < 8 || grad_stride % 4 != 0 ||
+        !aligned16(g_geometry))
+        return GSX_ERR_INVALID;
+    const bool inside = !g_features;  // the features' gradient follows in the record
+    if (inside ? grad_stride < 6 + C : feature_stride < C) return GSX_ERR_INVALID;
+    return raster_bwd(n, C, means2d, conic_opacity, features, sorted_ids, num_ids, tile_ranges,
+                      background, width, height, final_T, n_contrib, grad_out, grad_final_T,
+                      g_geometry, nullptr, g_features, nullptr, grad_stride,
+                      inside ? grad_stride : feature_stride, tile_order, stream);
 }
 
 int gsx_split_raster_grads(int64_t n, const float* record, int32_t grad_stride, float* g_means2d,

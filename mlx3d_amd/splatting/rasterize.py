@@ -116,26 +116,43 @@ def raster_backward(means2d, conic_opac, feats, sorted_ids, tile_ranges, backgro
     return g_m, g_c, g_f, g_o
 
 
+def _whole_lines(n: int, C: int, num_ids: int) -> bool:
+    """Whether the features' gradient is gathered in rows of whole 64-byte lines
+    and copied out of them: where the Gaussians reach six tiles or more on
+    average (below that the copy costs what the atomics save) and there are
+    half a million duplicates (below that they take less than the extra
+    calls' host time)."""
+    return 5 <= C <= 15 and num_ids >= max(6 * n, 1 << 19)
+
+
 def raster_backward_geometry(means2d, conic_opac, feats, sorted_ids, tile_ranges, background,
                              width, height, final_T, n_contrib, g_out, g_final_T,
                              tile_order=None):
-    """gsx_raster_bwd_geometry: (record (N, 8) = [means2d 2 | conic 3 | opacity
-    1 | padding], feature gradient (N, C)).  The geometric atomics of a Gaussian
-    share one cache line, which three arrays would spread over three."""
+    """The backward into (record (N, 8 or 16) = [means2d 2 | conic 3 | opacity 1 |
+    other words], feature gradient (N, C)).  The geometric atomics of a Gaussian
+    share one cache line, which three arrays would spread over three
+    (gsx_raster_bwd_geometry); where its features' would straddle lines they
+    lie in the record too, or in rows of 16 (gsx_raster_bwd_rows)."""
     dev = means2d.device
     n, C = feats.shape
-    rec = _empty((n, 8), dev)
-    g_f = _empty((n, C), dev)
+    rows = _whole_lines(n, C, sorted_ids.numel())
+    rec = _empty((n, 16 if rows and C <= 10 else 8), dev)
+    g_f = None if rows and C <= 10 else _empty((n, 16 if rows else C), dev)
     if g_out is None:
         g_out = torch.zeros((height, width, C), dtype=torch.float32, device=dev)
     g_out = _lib.f32c(g_out)
     g_final_T = None if g_final_T is None else _lib.f32c(g_final_T)
-    _lib.check(_lib.load().gsx_raster_bwd_geometry(
-        n, C, _lib.ptr(means2d), _lib.ptr(conic_opac), _lib.ptr(feats), _lib.ptr(sorted_ids),
-        sorted_ids.numel(), _lib.ptr(tile_ranges), _lib.ptr(background), width, height,
-        _lib.ptr(final_T), _lib.ptr(n_contrib), _lib.ptr(g_out), _lib.ptr(g_final_T),
-        _lib.ptr(rec), _lib.ptr(g_f), 8, _lib.ptr(tile_order), _lib.stream_handle(dev)),
-        "gsx_raster_bwd_geometry")
+    args = (n, C, _lib.ptr(means2d), _lib.ptr(conic_opac), _lib.ptr(feats), _lib.ptr(sorted_ids),
+            sorted_ids.numel(), _lib.ptr(tile_ranges), _lib.ptr(background), width, height,
+            _lib.ptr(final_T), _lib.ptr(n_contrib), _lib.ptr(g_out), _lib.ptr(g_final_T),
+            _lib.ptr(rec))
+    L, st = _lib.load(), _lib.stream_handle(dev)
+    if rows:
+        _lib.check(L.gsx_raster_bwd_rows(*args, rec.shape[1], _lib.ptr(g_f), 16,
+                                         _lib.ptr(tile_order), st), "gsx_raster_bwd_rows")
+        return rec, (rec[:, 6:6 + C] if g_f is None else g_f[:, :C]).contiguous()
+    _lib.check(L.gsx_raster_bwd_geometry(*args, _lib.ptr(g_f), 8, _lib.ptr(tile_order), st),
+               "gsx_raster_bwd_geometry")
     return rec, g_f
 
 

@@ -151,3 +151,22 @@ def test_no_kernel_spills_registers():
     assert len(usage) > 50
     spills = {k: v["ScratchSize"] for k, v in usage.items() if v.get("ScratchSize", 0)}
     assert not spills, spills
+
+
+def test_raster_bwd_rows_checks_its_layout():
+    """The spaced feature rows take 5 to 32 channels and strides that hold them."""
+    L = _lib.load()
+    buf = np.zeros(64, np.float32)
+    p = ctypes.c_void_p((buf.ctypes.data + 15) // 16 * 16)  # never dereferenced
+
+    def call(C, grad_stride, features, feature_stride, n=0, record=p):
+        return L.gsx_raster_bwd_rows(n, C, p, p, p, p, 0, p, None, 16, 16, p, p, p, None, record,
+                                     grad_stride, features, feature_stride, None, None)
+
+    assert call(5, 8, p, 16) == 0 and call(32, 40, None, 0) == 0
+    assert call(4, 8, p, 16) == -1 and call(33, 8, p, 48) == -1
+    assert call(12, 8, p, 11) == -1          # rows shorter than the channels
+    assert call(11, 16, None, 0) == -1       # a record that does not hold them
+    assert call(10, 16, None, 0) == 0
+    assert call(10, 7, p, 16) == -1 and call(10, 10, p, 16) == -1
+    assert call(10, 16, None, 0, record=ctypes.c_void_p(p.value + 4)) == -1

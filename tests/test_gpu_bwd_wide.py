@@ -5,6 +5,8 @@ its split form, against the oracle."""
 
 from __future__ import annotations
 
+import importlib
+
 import numpy as np
 import pytest
 import torch
@@ -14,6 +16,9 @@ from mlx3d_amd.splatting import bin_gaussians
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
+
+# the module (the package's attribute of that name is the function)
+RASTERIZE = importlib.import_module("mlx3d_amd.splatting.rasterize")
 
 
 def _scene(n, C, W, H, seed):
@@ -110,7 +115,9 @@ def _both(m2, con, op, feats, ids, ranges, W, H, bg, g_img, g_T):
                                        cu(g_img), cu(g_T))
     gm, gc, go = split_geometry(rec)
     got = {"means2d": gm, "conics": gc, "opacities": go, "features": gf}
-    assert float(rec[:, 6:].abs().max()) == 0.0
+    assert gf.is_contiguous()
+    if rec.shape[1] == 8:
+        assert float(rec[:, 6:].abs().max()) == 0.0
     return {k: (host(v), np.asarray(rg[k])) for k, v in got.items()}, ref["n_contrib"]
 
 
@@ -144,6 +151,42 @@ def _edges(n, C, W, H):
                                      (33, 33, 17, 9), (64, 34, 9, 17), (65, 36, 16, 16)])
 def test_wide_backward_list_edges(n, C, W, H):
     _edges(n, C, W, H)
+
+
+@pytest.mark.parametrize("n,C,W,H", [(1, 5, 1, 1), (17, 8, 7, 23), (81, 10, 33, 8),
+                                     (80, 11, 17, 15), (16, 15, 16, 16), (400, 10, 23, 9),
+                                     (400, 12, 23, 9)])
+def test_wide_backward_whole_lines(n, C, W, H, monkeypatch):
+    """The features' gradient gathered in the record or in rows of 16."""
+    monkeypatch.setattr(RASTERIZE, "_whole_lines", lambda n, C, d: True)
+    _edges(n, C, W, H)
+
+
+@pytest.mark.parametrize("C", [7, 13])
+def test_render_features_in_whole_lines(C, monkeypatch):
+    """A feature render whose Gaussians reach many tiles takes those rows by
+    itself and gives the gradients of the packed ones."""
+    from mlx3d_amd.cameras import Camera
+    from mlx3d_amd.splatting import render_gaussian_features
+
+    rng = np.random.default_rng(C)
+    n, W, H = 3000, 639, 361
+    raw = (rng.uniform(-1, 1, (n, 3)), rng.standard_normal((n, 4)),
+           rng.uniform(0.15, 0.4, (n, 3)), rng.uniform(0.01, 0.2, n), rng.standard_normal((n, C)))
+    cam = Camera.look_at(eye=(0, 0, -3.0), width=W, height=H)
+    g = cu(rng.standard_normal((H, W, C)).astype(np.float32))
+    taken, grads = [], []
+    rule = RASTERIZE._whole_lines
+    for force in (None, False):
+        monkeypatch.setattr(RASTERIZE, "_whole_lines", lambda *a, force=force: taken.append(
+            rule(*a) if force is None else force) or taken[-1])
+        t = [cu(np.asarray(a, np.float32)).requires_grad_(True) for a in raw]
+        render_gaussian_features(cam, *t)["features"].backward(g)
+        grads.append([host(x.grad) for x in t])
+    assert taken == [True, False]
+    for name, a, b in zip(("means", "quats", "scales", "opacities", "features"), *grads):
+        # the same sums, in the order the atomics came
+        np.testing.assert_allclose(a, b, rtol=0, atol=2e-5 * np.abs(b).max(), err_msg=name)
 
 
 @pytest.mark.parametrize("C", [6, 32])
