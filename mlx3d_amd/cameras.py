@@ -309,8 +309,11 @@ class Camera:
         # per field took 28 us of every render, this takes 8
         R = self.R.numpy().astype(np.float32).reshape(3, 3)
         t = self.t.numpy().astype(np.float32).reshape(3)
-        head = np.array((self.fx, self.fy, self.cx, self.cy, 1.3 * (0.5 * self.width / self.fx),
-                         1.3 * (0.5 * self.height / self.fy), self.znear), np.float32)
+        head = (self.fx, self.fy, self.cx, self.cy, 1.3 * (0.5 * self.width / self.fx),
+                1.3 * (0.5 * self.height / self.fy), self.znear)
+        if not all(isinstance(v, float) for v in head):  # an array of one element, say
+            head = [float(np.float32(v)) for v in head]
+        head = np.array(head, np.float32)
         tail = struct.pack("4i", int(self.width), int(self.height),
                            int(bool(self.orthographic)), self._lens_code())
         dist = bytes(32) if self.distortion is None else \

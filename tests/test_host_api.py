@@ -173,3 +173,35 @@ def test_adam_schedule_advances_only_after_launch():
     with pytest.raises(ValueError):  # CPU tensors are refused before any launch
         adam_step([(opt, {"p": torch.ones(8)}, {"p": p})])
     assert opt.step == 1 and opt.learning_rate == 1e-2
+
+
+def _cameras():
+    R, t = Camera.look_at(eye=(1.0, 2.0, -3.0), width=64, height=48).R, torch.tensor([0.1, -0.2, 3.0])
+    base = dict(R=R, t=t, fx=501.7, fy=499.3, cx=320.1, cy=239.9, width=641, height=479)
+    one = torch.tensor([0.1234567])
+    return {"pinhole": Camera(**base), "near": Camera(**base | dict(znear=0.0371)),
+            "ortho": Camera.orthographic_camera(1.7, 97, 55, R=R, t=t),
+            "brown4": Camera(**base, distortion=(0.1, -0.03, 1e-3, -2e-3)),
+            "brown5": Camera(**base, distortion=(0.1, -0.03, 1e-3, -2e-3, 0.017)),
+            "fisheye2": Camera(**base, distortion=(0.05, -0.02), fisheye=True),
+            "fisheye4": Camera(**base, distortion=(0.05, -0.02, 4e-3, -1e-3), fisheye=True),
+            "numpy": Camera(**base | dict(fx=np.float32(501.7), fy=np.float64(499.3),
+                                          width=np.int64(641), height=torch.tensor(479))),
+            "scalars": Camera(**base | dict(fx=torch.tensor(501.7), cx=torch.tensor(320.1))),
+            "one_element": Camera(**base | dict(fx=np.array([501.7]), cx=320.1 + 0 * one,
+                                                znear=one)),
+            "overflow": Camera(**base | dict(cx=1e39, cy=float("nan")))}
+
+
+@pytest.mark.filterwarnings("ignore:Conversion of an array", "ignore:overflow")
+@pytest.mark.parametrize("name", list(_cameras()))
+def test_camera_struct_holds_the_fields(name):
+    """The struct that the kernels read and the dict that the oracle reads hold the
+    same values, whatever kind of number an intrinsic is."""
+    cam = _cameras()[name]
+    f, g = cam.gsx_fields(), cam.to_gsx()
+    for k, want in f.items():
+        got = getattr(g, k)
+        got = list(got) if hasattr(got, "__len__") else got
+        np.testing.assert_array_equal(np.float32(got), np.float32(want).reshape(-1)
+                                      if np.ndim(want) else np.float32(want), err_msg=k)
