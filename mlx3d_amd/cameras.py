@@ -113,7 +113,7 @@ def look_at(eye, at, up) -> tuple[torch.Tensor, torch.Tensor]:
 
 def _center(R: np.ndarray, t: np.ndarray) -> np.ndarray:
     """-(R^T t) of float32 arrays, each component summed in index order."""
-    p = R * t[:, None]
+    p = R * t.reshape(3, 1)
     return -((p[0] + p[1]) + p[2])
 
 

@@ -205,3 +205,13 @@ def test_camera_struct_holds_the_fields(name):
         got = list(got) if hasattr(got, "__len__") else got
         np.testing.assert_array_equal(np.float32(got), np.float32(want).reshape(-1)
                                       if np.ndim(want) else np.float32(want), err_msg=k)
+
+
+def test_camera_center_of_a_column_translation():
+    """A translation assigned as a (3, 1) column has the centre of the (3,) one."""
+    cam = Camera.look_at(eye=(1.0, 2.0, -3.0), width=64, height=48)
+    want, fields = cam.camera_center, cam.gsx_fields()["center"]
+    cam.t = cam.t.reshape(3, 1)
+    assert cam.camera_center.shape == (3,) and torch.equal(cam.camera_center, want)
+    np.testing.assert_array_equal(cam.gsx_fields()["center"], fields)
+    assert list(cam.to_gsx().center) == [float(v) for v in fields]
