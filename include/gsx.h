@@ -365,8 +365,11 @@ int gsx_pack_conic_opacity(int64_t n, const float* conics,
  * (each XCD's contiguous band of tiles, longest lists first).  With
  * order_ready != 0 words [T, 2T) already hold that order, written by
  * gsx_bin_tiles_async for these ranges, which cleared words [0, T) too, and
- * the call only reads the order.  The
- * outputs do not depend on the order.  The buffer has no counterpart in the
+ * the call only reads the order.  Frames of up to 256 tiles raise the bounds
+ * with atomics: a second forward on the same ready order leaves the larger of
+ * both calls' bounds (a buffer whose order this call computes itself never
+ * does).  No output depends on the order or, in gsx_raster_bwd, on the bounds;
+ * they only balance the work.  The buffer has no counterpart in the
  * reference (whose Metal dispatch has no such control). */
 int gsx_raster_fwd(int64_t n, int32_t C, const float* means2d,
                    const float* conic_opacity, const float* features,
