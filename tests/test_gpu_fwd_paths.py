@@ -1,7 +1,8 @@
-"""The forward rasterizer's routes by frame size: frames of a few hundred tiles
-(one workgroup per quadrant), middle ones (the XCDs take the bands' lists in
-turns) and large ones.  One scene is drawn into canvases of every route; its
-pixels must be the same bits, whatever the canvas."""
+"""The forward rasterizer's routes: frames of up to 256 tiles (one workgroup per
+quadrant) and larger ones (the XCDs take the bands' lists in turns), whole and
+partial tiles and blocks of channels, plain and other batches.  One scene drawn
+into canvases of every size must have the same bits; frames of odd sizes, their
+edges covered, must have the oracle's."""
 
 import numpy as np
 import pytest
@@ -121,3 +122,47 @@ def test_channel_blocks_match_oracle(C):
     assert np.isinf(ref["image"][..., C - 1]).any()
     np.testing.assert_array_equal(host(nc), ref["n_contrib"])
     assert_features(host(out), ref["image"])
+
+
+# 943 tiles (7 past a multiple of 8), 273 tiles, 6363 tiles, a corner tile of 1 x 1
+@pytest.mark.parametrize("C,depth,W,H", [(1, True, 641, 359), (2, False, 641, 359),
+                                         (3, False, 641, 359), (3, True, 641, 359),
+                                         (4, True, 641, 359), (4, False, 331, 195),
+                                         (3, True, 1601, 1007), (1, False, 1601, 1007)])
+def test_render_of_odd_frames_matches_oracle(C, depth, W, H):
+    """Images, T, contributor counts, depth and gradients through the public render
+    (which takes the binning's order), Gaussians up to and past every edge."""
+    from gpu_util import assert_bits, cu, host, oracle_backward, oracle_forward, rel_err
+    from mlx3d_amd.cameras import Camera
+    from mlx3d_amd.splatting import render_gaussian_features
+
+    import torch
+
+    n = 4000
+    rng = np.random.default_rng(100 * C + W)
+    cam = Camera.look_at(eye=(0.0, 0.0, -4.0), width=W, height=H)
+    half = 4.0 * 0.5 * H / cam.fy  # of the frame's height in the plane of the means
+    f32 = lambda a: np.ascontiguousarray(a, np.float32)  # noqa: E731
+    means = f32(rng.uniform(-1.05, 1.05, (n, 3)) * [half * W / H, half, 0.5])
+    quats, scales = f32(rng.standard_normal((n, 4))), f32(rng.uniform(0.005, 0.06, (n, 3)))
+    opac, feats = f32(rng.uniform(0.02, 0.95, n)), f32(rng.standard_normal((n, C)))
+    bg = rng.random(C, dtype=np.float32)
+    t = [cu(a).requires_grad_(True) for a in (means, quats, scales, opac, feats)]
+    out = render_gaussian_features(cam, *t, background=cu(bg), return_depth=depth)
+    pre, f, ids, ranges, r = oracle_forward(cam, means, quats, scales, opac, colors=feats, bg=bg,
+                                            depth=depth)
+    nc = r["n_contrib"]
+    assert min(nc[0].max(), nc[-1].max(), nc[:, 0].max(), nc[:, -1].max()) > 0
+    np.testing.assert_array_equal(host(out["n_contrib"]), nc)
+    assert_bits(host(out["features"]), r["image"], "image")
+    assert_bits(host(out["final_T"]), r["final_T"], "final_T")
+    if depth:
+        assert_bits(host(out["depth"]), r["depth"], "depth")
+    g_img = rng.standard_normal((H, W, C)).astype(np.float32)
+    g_a = rng.standard_normal((H, W)).astype(np.float32)
+    torch.autograd.backward([out["features"], out["alpha"]], [cu(g_img), cu(g_a)])
+    g = oracle_backward(cam, means, quats, scales, opac, pre, f, ids, ranges, r, g_img, g_a, bg=bg)
+    for name, a in zip(("means", "quats", "scales", "opacities", "features"), t):
+        # float32 sums against float32 terms summed in 64 bits, each over up to
+        # the frame's pixels: the repository's bound for these gradients
+        assert rel_err(host(a.grad), g[name]) < 1e-3, name
