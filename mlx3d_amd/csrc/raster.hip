@@ -1,33 +1,36 @@
 // raster.hip -- tile compositing (replaces gs_rasterize_forward,
 // gs_rasterize_backward and gs_rasterize_depth, splatting/rasterize.py:28-290).
 //
-// One 256-lane workgroup (4 wave64) per 16x16 tile; wave w owns the 8x8
-// pixel quadrant (w&1, w>>1).  The tile's depth-sorted Gaussians are staged
-// through LDS in batches (two 16-byte records per Gaussian plus its
-// channels, read as broadcasts).  While staging, each lane tests its
-// Gaussian's alpha >= 1/255 ellipse against the four quadrants (exact
-// minimum of the conic form over each quadrant's pixel centres, with a
-// margin that covers the float32 rounding of the per-pixel power), and the
-// workgroup publishes per quadrant a bit mask of the Gaussians that can
-// touch it.  Each wave compacts its quadrant's bits into a list of record
-// offsets and walks it in list order, reading each Gaussian's records while
-// the previous one is evaluated.  Skipped pairs are exactly pairs whose
-// alpha is below 1/255, which the reference also skips, so every output is
-// unchanged.
+// Up to 16 channels the forward (k_raster_fwd) has one 256-lane workgroup (4
+// wave64) per 16x16 tile; wave w owns the 8x8 pixel quadrant (w&1, w>>1).  The
+// tile's depth-sorted Gaussians are staged through LDS in batches (16-byte
+// pieces, read as broadcasts).  While staging, each lane tests its Gaussian's
+// alpha >= 1/255 ellipse against the four quadrants (exact minimum of the conic
+// form over each quadrant's pixel centres, with a margin that covers the float32
+// rounding of the per-pixel power), and the workgroup publishes per quadrant a
+// bit mask of the Gaussians that can touch it.  Each wave compacts its
+// quadrant's bits into a list of record offsets and walks it in list order,
+// reading each Gaussian's records while the previous one is evaluated.  Skipped
+// pairs are exactly pairs whose alpha is below 1/255, which the reference also
+// skips, so every output is unchanged.
 //
 // Forward: per-pixel front-to-back compositing as rasterize.py:60-96 (same
 // skips, same termination before compositing the splat that would drop T
 // below 1e-4), branch-free per pair; a wave stops once its 64 pixels have
-// terminated and the workgroup stops loading once all 256 have.
+// terminated and the workgroup stops loading once all 256 have.  Small frames
+// give every quadrant a workgroup (k_raster_fwd_split: three waves evaluate
+// alphas, one composites); blocks of 17 to 32 channels form the channel sums on
+// the matrix cores (k_raster_fwd_mx).
 // Backward: back-to-front replay (rasterize.py:147-220) from the largest
 // n_contrib of each quadrant; the reference issues one atomic per (pixel,
-// Gaussian, component).  Up to four channels (k_raster_bwd) the lanes are
-// pixels: a pair's gradient terms are summed over the wave with cross-row
-// swaps and DPP row operations, two Gaussians per reduction, and after the
-// batch one lane per Gaussian adds the four waves' slots and issues one
-// global atomic per (Gaussian, tile, component).  From five channels on
-// (k_raster_bwd_wide) the lanes are Gaussians and the channel work runs on
-// the matrix cores.
+// Gaussian, component).  Up to four channels (k_raster_bwd) a workgroup has a
+// tile and its lanes are pixels: a pair's gradient terms are summed over the
+// wave with cross-row swaps and DPP row operations, two Gaussians per
+// reduction, and after the batch one lane per Gaussian adds the four waves'
+// slots and issues one global atomic per (Gaussian, tile, component).  From
+// five channels on (k_raster_bwd_wide) a workgroup is one wave with one
+// quadrant, the lanes are Gaussians and the channel work runs on the matrix
+// cores.
 #include <algorithm>
 #include <type_traits>
 
