@@ -302,8 +302,8 @@ int gsx_bin_sort_async(int64_t n, const uint32_t* tile_counts,
  * host_status != NULL (8 words) its last kernel writes the final status
  * there the same way.  tile_order: NULL, or the gsx_tile_order_words(W, H)
  * buffer of the frame's gsx_raster_fwd: the call writes the forward's tile
- * order for the ranges it produces into words [T, 2T) and clears the
- * bounds before them (the placement's
+ * order for the ranges it produces into words [T, 2T), the bands' list lengths
+ * behind it, and clears the bounds before it (the placement's
  * first workgroups compute it beside the placement; it is what
  * gsx_raster_fwd would compute), to be passed with order_ready = 1.
  *
@@ -362,11 +362,12 @@ int gsx_pack_conic_opacity(int64_t n, const float* conics,
  * int32 words that the call fills: words [0, T) (T = ceil(W/16)
  * ceil(H/16)) each tile's largest n_contrib, which gsx_raster_bwd orders
  * its tiles by; words [T, 2T) the order the workgroups take the tiles in
- * (each XCD's contiguous band of tiles, longest lists first).  With
- * order_ready != 0 words [T, 2T) already hold that order, written by
- * gsx_bin_tiles_async for these ranges, which cleared words [0, T) too, and
- * the call only reads the order.  Frames of up to 256 tiles raise the bounds
- * with atomics: a second forward on the same ready order leaves the larger of
+ * (each XCD's contiguous band of tiles, longest lists first) and, from 16
+ * tiles on, words [2T, 2T + 8) each band's longest list and [2T + 8, 2T + 16)
+ * the entries of its lists.  With order_ready != 0 words [T, 2T + 16) already
+ * hold these, written by gsx_bin_tiles_async for these ranges, which cleared
+ * words [0, T) too, and the call only reads them.  Frames of up to 512 tiles may
+ * raise the bounds with atomics: a second forward on the same ready order leaves the larger of
  * both calls' bounds (a buffer whose order this call computes itself never
  * does).  No output depends on the order or, in gsx_raster_bwd, on the bounds;
  * they only balance the work.  The buffer has no counterpart in the

@@ -609,38 +609,66 @@ __device__ __forceinline__ int fwd_channel(int i, int nc) {
     return CH <= 4 ? i : min(i & ~3, nc - 4) + (i & 3);
 }
 
-template <int CH, bool DEPTH>
-__global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
-    const float2* __restrict__ xy, const float4* __restrict__ co, const float* __restrict__ feat,
-    int C, int c0, int nc, const float* __restrict__ depths, const int* __restrict__ ids,
-    const int2* __restrict__ ranges, int64_t n, int64_t n_ids, const float* __restrict__ bg,
-    int W, int H, int tiles_x, float* __restrict__ out, float* __restrict__ final_T,
-    int* __restrict__ n_contrib, float* __restrict__ depth_out, float* __restrict__ alpha_out,
-    const int* __restrict__ order, int* __restrict__ work) {
-    constexpr int NV = CH + (DEPTH ? 1 : 0);
-    using Rec = FwdRec<NV>;
+// The arguments of the forward kernels up to 16 channels.
+struct FwdArgs {
+    const float2* xy;
+    const float4* co;
+    const float* feat;
+    int C, c0, nc;
+    const float* depths;
+    const int* ids;
+    const int2* ranges;
+    int64_t n, n_ids;
+    const float* bg;
+    int W, H, tiles_x;
+    float *out, *final_T;
+    int* n_contrib;
+    float *depth_out, *alpha_out;
+    int* work;
+};
+#define GSX_FWD_PARAMS                                                                            \
+    const float2 *__restrict__ xy, const float4 *__restrict__ co, const float *__restrict__ feat, \
+        int C, int c0, int nc, const float *__restrict__ depths, const int *__restrict__ ids,     \
+        const int2 *__restrict__ ranges, int64_t n, int64_t n_ids, const float *__restrict__ bg,  \
+        int W, int H, int tiles_x, float *__restrict__ out, float *__restrict__ final_T,          \
+        int *__restrict__ n_contrib, float *__restrict__ depth_out,                               \
+        float *__restrict__ alpha_out, const int *__restrict__ order, int *__restrict__ work
+#define GSX_FWD_ARGS                                                                              \
+    FwdArgs {                                                                                     \
+        xy, co, feat, C, c0, nc, depths, ids, ranges, n, n_ids, bg, W, H, tiles_x, out, final_T,  \
+            n_contrib, depth_out, alpha_out, work                                                 \
+    }
+
+template <int NV>
+struct FwdTileLds {
     // record kThreads is the lists' padding: opacity zero, which no pixel takes
-    __shared__ float4 s_rec[Rec::kPieces * kRecords];
-    __shared__ uint64_t s_mask[kWaves][kWaves];  // [quadrant][loader wave]
-    __shared__ uint32_t s_list[kWaves][kThreads + 8];  // walk lists (+ look-ahead room)
+    float4 rec[FwdRec<NV>::kPieces * kRecords];
+    uint64_t mask[kWaves][kWaves];  // [quadrant][loader wave]
     // one word per wave, written before a barrier and read by every thread
     // after it (a 16-byte read): some pixel of the wave still composites /
     // every Gaussian the wave staged is plain.  Each batch's reads come
     // before the next barrier, and the next batch writes only after it.
-    __shared__ __align__(16) uint32_t s_alive[kWaves];
-    __shared__ __align__(16) uint32_t s_plain[kWaves];
+    alignas(16) uint32_t alive[kWaves];
+    alignas(16) uint32_t plain[kWaves];
+    uint32_t list[kWaves][kThreads + 8];  // walk lists (+ look-ahead room)
+};
 
+// A tile by one workgroup, a wave per quadrant.
+template <int CH, bool DEPTH>
+__device__ __forceinline__ void fwd_tile(FwdTileLds<CH + (DEPTH ? 1 : 0)>& s, int tile,
+                                         const FwdArgs& A) {
+    constexpr int NV = CH + (DEPTH ? 1 : 0);
+    using Rec = FwdRec<NV>;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tile = __builtin_amdgcn_readfirstlane(tile_at(order, blockIdx.x, gridDim.x, false));
-    const int tx = tile % tiles_x, ty = tile / tiles_x;
+    const int tx = tile % A.tiles_x, ty = tile / A.tiles_x;
     const int px0 = tx * kTile, py0 = ty * kTile;
     const int px = px0 + (wave & 1) * 8 + (lane & 7);
     const int py = py0 + (wave >> 1) * 8 + (lane >> 3);
-    const bool inside = px < W && py < H;
+    const bool inside = px < A.W && py < A.H;
 
     int start, num;
-    tile_span(ranges[tile], n_ids, start, num);
+    tile_span(A.ranges[tile], A.n_ids, start, num);
 
     FwdPixel<NV> p;
     p.x = (float)px + 0.5f;
@@ -652,32 +680,32 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
     uint64_t alive = __ballot(inside);  // the wave's pixels still compositing
     // the padding record (written before the first barrier)
     if (tid < Rec::kPieces)
-        s_rec[tid * kRecords + kThreads] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        s.rec[tid * kRecords + kThreads] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 
     for (int base = 0; base < num; base += kThreads) {
         const int lane = lane_again(), tid = wave * kWave + lane;
-        if (lane == 0) s_alive[wave] = alive != 0ull;
+        if (lane == 0) s.alive[wave] = alive != 0ull;
         __syncthreads();
-        const uint4 al = *reinterpret_cast<const uint4*>(s_alive);
+        const uint4 al = *reinterpret_cast<const uint4*>(s.alive);
         if ((al.x | al.y | al.z | al.w) == 0u) break;  // all 256 pixels done
         const int k = base + tid;
         uint32_t qm = 0;
         bool plain = true;
         if (k < num) {
-            const int g = ids[start + k];
-            if ((uint32_t)g < (uint64_t)n) {
+            const int g = A.ids[start + k];
+            if ((uint32_t)g < (uint64_t)A.n) {
                 // the record, depth and feature loads issue together
-                const float2 m = xy[g];
-                const float4 c = co[g];
+                const float2 m = A.xy[g];
+                const float4 c = A.co[g];
                 float v[4 * Rec::X4 + 2];
 #pragma unroll
                 for (int i = 0; i < 4 * Rec::X4 + 2; ++i) v[i] = 0.0f;
-                const float* const f = feat + (int64_t)g * C + c0;
+                const float* const f = A.feat + (int64_t)g * A.C + A.c0;
 #pragma unroll
-                for (int i = 0; i < CH; ++i) v[i] = f[fwd_channel<CH>(i, nc)];
-                if (DEPTH) v[CH] = depths[g];
+                for (int i = 0; i < CH; ++i) v[i] = f[fwd_channel<CH>(i, A.nc)];
+                if (DEPTH) v[CH] = A.depths[g];
                 const float thr = alpha_floor_power(c.w);
-                float4* const r = s_rec + tid;
+                float4* const r = s.rec + tid;
                 r[0] = make_float4(m.x, m.y, c.w, v[0]);
                 r[kRecords] = make_float4(-0.5f * c.x, -c.y, -0.5f * c.z, v[1]);
 #pragma unroll
@@ -693,43 +721,50 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(
 #pragma unroll
         for (int q = 0; q < kWaves; ++q) {
             const uint64_t b = __ballot((qm >> q) & 1u);
-            if (lane == 0) s_mask[q][wave] = b;
+            if (lane == 0) s.mask[q][wave] = b;
         }
         const uint64_t np = __ballot(!plain);
-        if (lane == 0) s_plain[wave] = np == 0ull;
+        if (lane == 0) s.plain[wave] = np == 0ull;
         __syncthreads();
-        const uint4 pl = *reinterpret_cast<const uint4*>(s_plain);
+        const uint4 pl = *reinterpret_cast<const uint4*>(s.plain);
         const bool batch_plain = (pl.x & pl.y & pl.z & pl.w) != 0u;
         if (alive == 0ull) continue;
         const int cnt =
-            build_list<kWaves, false, 4>(s_mask[wave], s_list[wave], lane, 16, kThreads);
+            build_list<kWaves, false, 4>(s.mask[wave], s.list[wave], lane, 16, kThreads);
         p.last_off = -1;
         if (batch_plain)
-            fwd_walk<NV, true>(s_list[wave], cnt, s_rec, p, alive);
+            fwd_walk<NV, true>(s.list[wave], cnt, s.rec, p, alive);
         else
-            fwd_walk<NV, false>(s_list[wave], cnt, s_rec, p, alive);
+            fwd_walk<NV, false>(s.list[wave], cnt, s.rec, p, alive);
         if (p.last_off >= 0) last = base + (p.last_off >> 4) + 1;
     }
     if (inside) {
-        const int64_t pid = (int64_t)py * W + px;
+        const int64_t pid = (int64_t)py * A.W + px;
         const float T = p.T;
-        float* o = out + pid * C + c0;
+        float* o = A.out + pid * A.C + A.c0;
 #pragma unroll
         for (int i = 0; i < CH; ++i) {
-            const int ch = fwd_channel<CH>(i, nc);
-            o[ch] = p.acc[i] + T * (bg ? bg[c0 + ch] : 0.0f);
+            const int ch = fwd_channel<CH>(i, A.nc);
+            o[ch] = p.acc[i] + T * (A.bg ? A.bg[A.c0 + ch] : 0.0f);
         }
-        if (c0 == 0) {
-            final_T[pid] = T;
-            n_contrib[pid] = last;
-            if (alpha_out) alpha_out[pid] = 1.0f - T;
+        if (A.c0 == 0) {
+            A.final_T[pid] = T;
+            A.n_contrib[pid] = last;
+            if (A.alpha_out) A.alpha_out[pid] = 1.0f - T;
             if (DEPTH) {
                 const float al = 1.0f - T;
-                depth_out[pid] = al > 1e-6f ? p.acc[CH] / al : 0.0f;
+                A.depth_out[pid] = al > 1e-6f ? p.acc[CH] / al : 0.0f;
             }
         }
     }
-    if (work) store_tile_work(work, tile, last, wave, lane);
+    if (A.work) store_tile_work(A.work, tile, last, wave, lane);
+}
+
+template <int CH, bool DEPTH>
+__global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(GSX_FWD_PARAMS) {
+    __shared__ FwdTileLds<CH + (DEPTH ? 1 : 0)> s;
+    const int tile = __builtin_amdgcn_readfirstlane(tile_at(order, blockIdx.x, gridDim.x, false));
+    fwd_tile<CH, DEPTH>(s, tile, GSX_FWD_ARGS);
 }
 
 // The forward of small frames.  One wave composites a quadrant's list serially
@@ -747,44 +782,39 @@ constexpr int kSplitChunk = kSplitWaves * kSplitPart;
 constexpr int kSplitRead = 8;                     // entries composited per round of reads
 static_assert(kSplitPart % kSplitRead == 0, "a round lies in one wave's part");
 
-template <int CH, bool DEPTH>
-__global__ __launch_bounds__(kThreads) void k_raster_fwd_split(
-    const float2* __restrict__ xy, const float4* __restrict__ co, const float* __restrict__ feat,
-    int C, int nc, const float* __restrict__ depths, const int* __restrict__ ids,
-    const int2* __restrict__ ranges, int64_t n, int64_t n_ids, const float* __restrict__ bg,
-    int W, int H, int tiles_x, int tiles, float* __restrict__ out, float* __restrict__ final_T,
-    int* __restrict__ n_contrib, float* __restrict__ depth_out, float* __restrict__ alpha_out,
-    const int* __restrict__ order, int* __restrict__ work) {
-    constexpr int NV = CH + (DEPTH ? 1 : 0);
-    constexpr int V4 = (NV + 3) / 4;
-    static_assert(kThreads == (kSplitWaves + 1) * kWave, "one compositing wave");
+template <int NV>
+struct FwdQuadLds {
+    static constexpr int V4 = (NV + 3) / 4;
     // the batch's entries that reach the quadrant, in list order
-    __shared__ float4 s_r0[kThreads];       // mean x, mean y, opacity, list position (int bits)
-    __shared__ float4 s_r1[kThreads];       // -a/2, -b, -c/2, log-alpha bound
-    __shared__ float4 s_v[kThreads][V4];    // channels, then depth
-    __shared__ float s_alpha[2][kSplitChunk][kWave];
-    __shared__ int s_cnt[kWaves];
-    __shared__ uint32_t s_plain[kWaves];
+    float4 r0[kThreads];     // mean x, mean y, opacity, list position (int bits)
+    float4 r1[kThreads];     // -a/2, -b, -c/2, log-alpha bound
+    float4 v[kThreads][V4];  // channels, then depth
+    float alpha[2][kSplitChunk][kWave];
+    int cnt[kWaves];
+    uint32_t plain[kWaves];
     // chunk c's word c & 1: every pixel has stopped.  Written before the
     // chunk's barrier and read after it; the next write of the word follows
     // the next chunk's barrier, which every reader has reached.
-    __shared__ uint32_t s_stop[2];
+    uint32_t stop[2];
+};
 
-    // workgroups 32 i + 8 q + x: quadrant q of the tile in slot 8 i + x
-    const uint32_t bid = blockIdx.x;
-    const int slot = (int)((bid & 7u) | ((bid >> 5) << 3)), quad = (int)(bid >> 3) & 3;
-    if (slot >= tiles) return;
+// A quadrant of a tile by one workgroup.
+template <int CH, bool DEPTH>
+__device__ __forceinline__ void fwd_quadrant(FwdQuadLds<CH + (DEPTH ? 1 : 0)>& s, int tile,
+                                             int quad, const FwdArgs& A) {
+    constexpr int NV = CH + (DEPTH ? 1 : 0);
+    constexpr int V4 = (NV + 3) / 4;
+    static_assert(kThreads == (kSplitWaves + 1) * kWave, "one compositing wave");
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tile = __builtin_amdgcn_readfirstlane(tile_at(order, slot, tiles, false));
-    const int qx0 = (tile % tiles_x) * kTile + (quad & 1) * 8;
-    const int qy0 = (tile / tiles_x) * kTile + (quad >> 1) * 8;
+    const int qx0 = (tile % A.tiles_x) * kTile + (quad & 1) * 8;
+    const int qy0 = (tile / A.tiles_x) * kTile + (quad >> 1) * 8;
     const int px = qx0 + (lane & 7), py = qy0 + (lane >> 3);
-    const bool inside = px < W && py < H;
+    const bool inside = px < A.W && py < A.H;
     const float pxf = (float)px + 0.5f, pyf = (float)py + 0.5f;
 
     int start, num;
-    tile_span(ranges[tile], n_ids, start, num);
+    tile_span(A.ranges[tile], A.n_ids, start, num);
 
     // wave 0's pixels
     float T = 1.0f, acc[NV];
@@ -803,15 +833,15 @@ __global__ __launch_bounds__(kThreads) void k_raster_fwd_split(
 #pragma unroll
         for (int i = 0; i < 4 * V4; ++i) v[i] = 0.0f;
         if (k < num) {
-            const int g = ids[start + k];
-            if ((uint32_t)g < (uint64_t)n) {
+            const int g = A.ids[start + k];
+            if ((uint32_t)g < (uint64_t)A.n) {
                 // the record, depth and feature loads issue together
-                m = xy[g];
-                c = co[g];
-                const float* const f = feat + (int64_t)g * C;
+                m = A.xy[g];
+                c = A.co[g];
+                const float* const f = A.feat + (int64_t)g * A.C;
 #pragma unroll
                 for (int ch = 0; ch < CH; ++ch) v[ch] = f[ch];  // CH == nc == C
-                if (DEPTH) v[CH] = depths[g];
+                if (DEPTH) v[CH] = A.depths[g];
                 keep = quadrant_reached(m.x, m.y, c, qx0, qy0);
                 thr = alpha_floor_power(c.w);
                 plain = plain_gaussian<0>(m.x, m.y, c, thr, nullptr);
@@ -821,25 +851,25 @@ __global__ __launch_bounds__(kThreads) void k_raster_fwd_split(
         }
         const uint64_t kept = __ballot(keep), odd = __ballot(keep && !plain);
         if (lane == 0) {
-            s_cnt[wave] = __popcll(kept);
-            s_plain[wave] = odd == 0ull;
+            s.cnt[wave] = __popcll(kept);
+            s.plain[wave] = odd == 0ull;
         }
         __syncthreads();
         int cnt = 0, at = __popcll(kept & ((1ull << lane) - 1ull));
         bool batch_plain = true;
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
-            if (w < wave) at += s_cnt[w];
-            cnt += s_cnt[w];
-            batch_plain = batch_plain && s_plain[w] != 0u;
+            if (w < wave) at += s.cnt[w];
+            cnt += s.cnt[w];
+            batch_plain = batch_plain && s.plain[w] != 0u;
         }
         cnt = __builtin_amdgcn_readfirstlane(cnt);
         if (keep) {
-            s_r0[at] = make_float4(m.x, m.y, c.w, __int_as_float(k));
-            s_r1[at] = make_float4(-0.5f * c.x, -c.y, -0.5f * c.z, thr);
+            s.r0[at] = make_float4(m.x, m.y, c.w, __int_as_float(k));
+            s.r1[at] = make_float4(-0.5f * c.x, -c.y, -0.5f * c.z, thr);
 #pragma unroll
             for (int i = 0; i < V4; ++i)
-                s_v[at][i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+                s.v[at][i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
         }
         __syncthreads();
         const int chunks = (cnt + kSplitChunk - 1) / kSplitChunk;
@@ -850,7 +880,7 @@ __global__ __launch_bounds__(kThreads) void k_raster_fwd_split(
 #pragma unroll 4
                     for (int j = 0; j < kSplitPart; ++j) {
                         const int e = min(e0 + j, cnt - 1);  // past the end: alpha zero
-                        const float4 r0 = s_r0[e], r1 = s_r1[e];
+                        const float4 r0 = s.r0[e], r1 = s.r1[e];
                         const float power =
                             splat_power(r1.x, r1.y, r1.z, r0.x - pxf, r0.y - pyf);
                         const bool ok = batch_plain ? !(power < -86.0f)
@@ -859,14 +889,14 @@ __global__ __launch_bounds__(kThreads) void k_raster_fwd_split(
                             batch_plain ? splat_exp_core(power) : splat_exp_sel(power);
                         const float alpha = fminf(0.99f, r0.z * ex);
                         const bool take = ok && !(alpha < 1.0f / 255.0f) && e0 + j < cnt;
-                        s_alpha[ck & 1][j0 + j][lane] = take ? alpha : 0.0f;
+                        s.alpha[ck & 1][j0 + j][lane] = take ? alpha : 0.0f;
                     }
                 }
             } else {
                 if (ck > 0) {
                     const int f0 = (ck - 1) * kSplitChunk;
                     const int len = min(kSplitChunk, cnt - f0);
-                    const float(*const sa)[kWave] = s_alpha[(ck - 1) & 1];
+                    const float(*const sa)[kWave] = s.alpha[(ck - 1) & 1];
                     int at_last = -1;
                     auto entry = [&](int j, float a, const float4* val, bool masked) {
                         const float next_T = T * (1.0f - a);
@@ -879,8 +909,8 @@ __global__ __launch_bounds__(kThreads) void k_raster_fwd_split(
                         at_last = w > 0.0f ? j : at_last;
 #pragma unroll
                         for (int i = 0; i < NV; ++i) {
-                            const float s = fmaf(comp4(val[i >> 2], i & 3), w, acc[i]);
-                            acc[i] = (!masked || w > 0.0f) ? s : acc[i];
+                            const float sum = fmaf(comp4(val[i >> 2], i & 3), w, acc[i]);
+                            acc[i] = (!masked || w > 0.0f) ? sum : acc[i];
                         }
                     };
                     if (batch_plain) {
@@ -894,7 +924,7 @@ __global__ __launch_bounds__(kThreads) void k_raster_fwd_split(
                                 a[u] = sa[j + u][lane];
 #pragma unroll
                                 for (int i = 0; i < V4; ++i)
-                                    val[u][i] = s_v[min(f0 + j + u, cnt - 1)][i];
+                                    val[u][i] = s.v[min(f0 + j + u, cnt - 1)][i];
                             }
 #pragma unroll
                             for (int u = 0; u < kSplitRead; ++u)
@@ -902,50 +932,107 @@ __global__ __launch_bounds__(kThreads) void k_raster_fwd_split(
                         }
                     } else {
 #pragma unroll 1
-                        for (int j = 0; j < len; ++j) entry(j, sa[j][lane], s_v[f0 + j], true);
+                        for (int j = 0; j < len; ++j) entry(j, sa[j][lane], s.v[f0 + j], true);
                     }
-                    if (at_last >= 0) last = __float_as_int(s_r0[f0 + at_last].w) + 1;
+                    if (at_last >= 0) last = __float_as_int(s.r0[f0 + at_last].w) + 1;
                 }
-                if (lane == 0) s_stop[ck & 1] = alive == 0ull;
+                if (lane == 0) s.stop[ck & 1] = alive == 0ull;
             }
             __syncthreads();
-            stopped = s_stop[ck & 1] != 0u;
+            stopped = s.stop[ck & 1] != 0u;
             if (stopped) break;
         }
     }
     if (wave > 0) return;
     if (inside) {
-        const int64_t pid = (int64_t)py * W + px;
-        float* o = out + pid * C;
+        const int64_t pid = (int64_t)py * A.W + px;
+        float* o = A.out + pid * A.C;
 #pragma unroll
         for (int ch = 0; ch < CH; ++ch)
-            if (ch < nc) o[ch] = acc[ch] + T * (bg ? bg[ch] : 0.0f);
-        final_T[pid] = T;
-        n_contrib[pid] = last;
-        if (alpha_out) alpha_out[pid] = 1.0f - T;
+            o[ch] = acc[ch] + T * (A.bg ? A.bg[ch] : 0.0f);
+        A.final_T[pid] = T;
+        A.n_contrib[pid] = last;
+        if (A.alpha_out) A.alpha_out[pid] = 1.0f - T;
         if (DEPTH) {
             const float al = 1.0f - T;
-            depth_out[pid] = al > 1e-6f ? acc[CH] / al : 0.0f;
+            A.depth_out[pid] = al > 1e-6f ? acc[CH] / al : 0.0f;
         }
     }
-    if (work) {
+    if (A.work) {
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) last = max(last, __shfl_xor(last, o, kWave));
-        if (lane == 0) atomicMax(&work[tile], last);  // cleared with the order
+        if (lane == 0) atomicMax(&A.work[tile], last);  // cleared with the order
     }
+}
+
+template <int CH, bool DEPTH>
+__global__ __launch_bounds__(kThreads) void k_raster_fwd_split(GSX_FWD_PARAMS, int tiles) {
+    __shared__ FwdQuadLds<CH + (DEPTH ? 1 : 0)> s;
+    // workgroups 32 i + 8 q + x: quadrant q of the tile in slot 8 i + x
+    const uint32_t bid = blockIdx.x;
+    const int slot = (int)((bid & 7u) | ((bid >> 5) << 3)), quad = (int)(bid >> 3) & 3;
+    if (slot >= tiles) return;
+    const int tile = __builtin_amdgcn_readfirstlane(tile_at(order, slot, tiles, false));
+    fwd_quadrant<CH, DEPTH>(s, tile, quad, GSX_FWD_ARGS);
 }
 
 // Frames up to this many tiles take k_raster_fwd_split: all of its four workgroups
 // per tile then have a place at once on 256 compute units, whose LDS holds four
-// each (37 KB up to four values), or three (41 KB).  In two rounds it loses
-// wherever the work is spread over the frame, and splitting only as many of the
-// longest lists as leave every workgroup a place still lost up to 25 % there.
-// k_raster_fwd -> k_raster_fwd_split, us, for 10k in a blob, 300k in a box, 1M
-// on shells, 400k with heavy tails: 110 tiles 153 -> 121, 268 -> 184, 169 -> 143,
-// 39 -> 35; 169 tiles 128 -> 103, 176 -> 130, 138 -> 125, 33 -> 34; 256 tiles
-// 106 -> 87, 123 -> 97, 114 -> 102, 31 -> 31; 342 tiles 101 -> 83, 113 -> 96,
-// 110 -> 136, 30 -> 45; 510 tiles 104 -> 85, 129 -> 103, 113 -> 145, 32 -> 53.
+// each (37 KB up to four values), or three (41 KB).  k_raster_fwd ->
+// k_raster_fwd_split, us, for 10k in a blob, 300k in a box, 1M on shells, 400k
+// with heavy tails: 110 tiles 153 -> 121, 268 -> 184, 169 -> 143, 39 -> 35; 169
+// tiles 128 -> 103, 176 -> 130, 138 -> 125, 33 -> 34; 256 tiles 106 -> 87, 123 ->
+// 97, 114 -> 102, 31 -> 31.
 constexpr int split_tiles(int values) { return values <= 4 ? 256 : 192; }
+
+// Beyond that, up to this many, they run in two rounds, which a frame bound by a
+// few crowded tiles gains from and an evenly filled one does not: 342 tiles, the
+// same scenes, 101 -> 83, 113 -> 96, 110 -> 136, 30 -> 45; 510 tiles 104 -> 85,
+// 129 -> 103, 113 -> 145, 32 -> 53.  The workgroups decide by how far the longest
+// list exceeds the mean one (the order's builders leave both, per band): from
+// eight times on every scene gains (blobs, 10 to 20 times, a fifth).  Between 3.2
+// and 8 times (boxes, shells on a wide frame) those gain, up to a seventh, whose
+// mean list is short; past about 1500 entries the lists are mostly entries that no
+// pixel gets to and every quadrant stages them (1M on shells, 3.9 times, mean 4084: 107
+// -> 150).  Below (heavy tails, shells) most lose, 51 us instead of 29 at
+// worst.  With the values that leave room for three workgroups only the crowded
+// frames gain.
+constexpr int kChooseTiles = 512;
+__device__ __forceinline__ bool crowded(const int* bands, int tiles, bool narrow) {
+    int64_t longest = 0, entries = 0;
+#pragma unroll
+    for (int x = 0; x < kOrderBands; ++x) {
+        longest = max(longest, (int64_t)bands[x]);
+        entries += (uint32_t)bands[kOrderBands + x];
+    }
+    longest *= tiles;
+    return longest >= 8 * entries ||
+           (narrow && 5 * longest >= 16 * entries && entries <= (int64_t)1500 * tiles);
+}
+
+template <int NV>
+union FwdChooseLds {
+    FwdTileLds<NV> tile;
+    FwdQuadLds<NV> quad;
+};
+
+template <int CH, bool DEPTH>
+__global__ __launch_bounds__(kThreads) void k_raster_fwd_choose(GSX_FWD_PARAMS, int tiles) {
+    constexpr int NV = CH + (DEPTH ? 1 : 0);
+    __shared__ FwdChooseLds<NV> s;
+    // each XCD's tiles with their first workgroup, then the other three
+    const int x = (int)blockIdx.x & 7, j = (int)blockIdx.x >> 3, per = (tiles + 7) / 8;
+    const int rank = j < per ? j : (j - per) / 3, quad = j < per ? 0 : 1 + (j - per) % 3;
+    const int slot = 8 * rank + x;
+    if (slot >= tiles) return;
+    const bool split = crowded(order + tiles, tiles, NV <= 4);
+    if (!split && quad != 0) return;
+    const int tile = __builtin_amdgcn_readfirstlane(tile_at(order, slot, tiles, false));
+    if (split)
+        fwd_quadrant<CH, DEPTH>(s.quad, tile, quad, GSX_FWD_ARGS);
+    else
+        fwd_tile<CH, DEPTH>(s.tile, tile, GSX_FWD_ARGS);
+}
 
 // Per-pixel state of the back-to-front replay.
 //
@@ -2530,16 +2617,16 @@ void launch_fwd(dim3 grid, hipStream_t st, bool depth, const float2* xy, const f
         return;
     }
     if constexpr (CH <= 4) {
-        if ((int)grid.x <= split_tiles(CH + (depth ? 1 : 0)) && C <= 4) {
-            const dim3 wgs(32u * ((grid.x + 7u) / 8u));
-            if (depth)
-                hipLaunchKernelGGL((k_raster_fwd_split<CH, true>), wgs, dim3(kThreads), 0, st, xy,
-                                   co, feat, C, nc, depths, ids, ranges, n, n_ids, bg, W, H,
-                                   tiles_x, (int)grid.x, out, fT, ncon, dout, aout, order, work);
-            else
-                hipLaunchKernelGGL((k_raster_fwd_split<CH, false>), wgs, dim3(kThreads), 0, st,
-                                   xy, co, feat, C, nc, depths, ids, ranges, n, n_ids, bg, W, H,
-                                   tiles_x, (int)grid.x, out, fT, ncon, dout, aout, order, work);
+        const int tiles = (int)grid.x;
+        const bool all = tiles <= split_tiles(CH + (depth ? 1 : 0));
+        if (C <= 4 && (all || (order && tiles <= kChooseTiles))) {
+            auto* const kernel = all ? (depth ? k_raster_fwd_split<CH, true>
+                                              : k_raster_fwd_split<CH, false>)
+                                     : (depth ? k_raster_fwd_choose<CH, true>
+                                              : k_raster_fwd_choose<CH, false>);
+            hipLaunchKernelGGL(kernel, dim3(32u * (((unsigned)tiles + 7u) / 8u)), dim3(kThreads),
+                               0, st, xy, co, feat, C, c0, nc, depths, ids, ranges, n, n_ids, bg,
+                               W, H, tiles_x, out, fT, ncon, dout, aout, order, work, tiles);
             return;
         }
     }

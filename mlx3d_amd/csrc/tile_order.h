@@ -21,7 +21,9 @@ __device__ __forceinline__ void tile_span(int2 rg, int64_t n_ids, int& start, in
 // descending quarter-octave bucket of the estimate (4 log2(w + 1), 64
 // buckets) with a counting sort.  Forward (BWD false): the estimate is the
 // list length (ranges), the bands are xcd_remap's (equal tile counts), and
-// tile t lands at order[band start + its rank in the band].  Backward: the
+// tile t lands at order[band start + its rank in the band]; from 16 tiles on the
+// band's longest list goes to order[T + band] and the number of its lists'
+// entries to order[T + 8 + band].  Backward: the
 // estimate is the contributor bound the forward stored (work, the entries
 // the backward replays); up to 16384 tiles the bands are cut at equal
 // shares of sum(min(w, 2^16) + 16) (the 16 stands for a tile's fixed cost;
@@ -159,6 +161,8 @@ __device__ __forceinline__ void tile_order_band(int band, const int2* __restrict
     // similar work run close together in time and share the XCD's L2.
     // Bands of more than kBandItems * 1024 tiles are placed in rounds, each
     // round sorted on its own (the rounds in raster order).
+    int longest = 0;        // of the thread's tiles
+    uint32_t entries = 0u;  // (wraps for ranges that overlap)
     for (int r0 = lo; r0 < hi; r0 += kBandItems * THREADS) {
         int bk[kBandItems], est[kBandItems];
         uint32_t rk[kBandItems];
@@ -169,6 +173,10 @@ __device__ __forceinline__ void tile_order_band(int band, const int2* __restrict
         for (int k = 0; k < kBandItems; ++k) {
             const int t = r0 + k * THREADS + tid;
             bk[k] = t < hi ? order_bucket(est[k]) : -1;
+            if (!BWD && t < hi) {
+                longest = max(longest, est[k]);
+                entries += (uint32_t)est[k];
+            }
         }
 #pragma unroll
         for (int k = 0; k < kBandItems; ++k) {
@@ -224,6 +232,29 @@ __device__ __forceinline__ void tile_order_band(int band, const int2* __restrict
              k += THREADS)
             s_cnt[k] = 0u;
         __syncthreads();
+    }
+    // the band's longest list and its entries, behind the T order words
+    if (!BWD && tiles >= 2 * kOrderBands) {
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) {
+            longest = max(longest, __shfl_xor(longest, o, kWave));
+            entries += __shfl_xor(entries, o, kWave);
+        }
+        if (lane == 0) {
+            s_cnt[wave] = (uint32_t)longest;
+            s_cnt[THREADS / kWave + wave] = entries;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            int l = 0;
+            uint32_t e = 0u;
+            for (int x = 0; x < THREADS / kWave; ++x) {
+                l = max(l, (int)s_cnt[x]);
+                e += s_cnt[THREADS / kWave + x];
+            }
+            order[tiles + band] = l;
+            order[tiles + kOrderBands + band] = (int)e;
+        }
     }
 }
 

@@ -1,6 +1,6 @@
 """The forward rasterizer's routes: frames of up to 256 tiles (one workgroup per
-quadrant) and larger ones (the XCDs take the bands' lists in turns), whole and
-partial tiles and blocks of channels, plain and other batches.  One scene drawn
+quadrant), up to 512 (the same where a few tiles are crowded, by the lists'
+lengths beside the order) and larger ones, whole and partial tiles and blocks of channels, plain and other batches.  One scene drawn
 into canvases of every size must have the same bits; frames of odd sizes, their
 edges covered, must have the oracle's."""
 
@@ -49,7 +49,7 @@ def _frame(W, H, C, depth, plain, n=900):
                                            (3, True, True), (4, True, True), (3, True, False),
                                            (5, False, True), (16, True, True)])
 def test_frame_sizes_agree(C, depth, plain):
-    # 30, 192 | 208, 256 | 272, 396, 525, 3600, 6500 tiles
+    # 30, 192 | 208, 256 | 272, 396 | 525, 3600, 6500 tiles
     base, bounds = _frame(96, 80, C, depth, plain)
     n_contrib = base[2]
     tiles = n_contrib.reshape(5, 16, 6, 16).max(axis=(1, 3))
@@ -124,12 +124,15 @@ def test_channel_blocks_match_oracle(C):
     assert_features(host(out), ref["image"])
 
 
-# 943 tiles (7 past a multiple of 8), 273 tiles, 6363 tiles, a corner tile of 1 x 1
-@pytest.mark.parametrize("C,depth,W,H", [(1, True, 641, 359), (2, False, 641, 359),
-                                         (3, False, 641, 359), (3, True, 641, 359),
-                                         (4, True, 641, 359), (4, False, 331, 195),
-                                         (3, True, 1601, 1007), (1, False, 1601, 1007)])
-def test_render_of_odd_frames_matches_oracle(C, depth, W, H):
+# 943 tiles (7 past a multiple of 8), 273, 294, 209 and 6363 tiles, corner tiles of
+# 1 x 1; 273 to 294 tiles evenly filled and crowded
+@pytest.mark.parametrize("C,depth,W,H,crowd", [
+    (1, True, 641, 359, False), (2, False, 641, 359, False), (3, False, 641, 359, False),
+    (3, True, 641, 359, False), (4, True, 641, 359, True), (4, False, 331, 195, False),
+    (4, False, 331, 195, True), (1, True, 331, 195, True), (4, True, 289, 167, False),
+    (4, True, 289, 167, True), (2, False, 335, 211, True), (3, True, 335, 211, False),
+    (3, True, 335, 211, True), (3, True, 1601, 1007, False), (1, False, 1601, 1007, True)])
+def test_render_of_odd_frames_matches_oracle(C, depth, W, H, crowd):
     """Images, T, contributor counts, depth and gradients through the public render
     (which takes the binning's order), Gaussians up to and past every edge."""
     from gpu_util import assert_bits, cu, host, oracle_backward, oracle_forward, rel_err
@@ -144,6 +147,8 @@ def test_render_of_odd_frames_matches_oracle(C, depth, W, H):
     half = 4.0 * 0.5 * H / cam.fy  # of the frame's height in the plane of the means
     f32 = lambda a: np.ascontiguousarray(a, np.float32)  # noqa: E731
     means = f32(rng.uniform(-1.05, 1.05, (n, 3)) * [half * W / H, half, 0.5])
+    if crowd:
+        means[n // 4:, :2] *= np.float32(0.04)
     quats, scales = f32(rng.standard_normal((n, 4))), f32(rng.uniform(0.005, 0.06, (n, 3)))
     opac, feats = f32(rng.uniform(0.02, 0.95, n)), f32(rng.standard_normal((n, C)))
     bg = rng.random(C, dtype=np.float32)
@@ -151,7 +156,8 @@ def test_render_of_odd_frames_matches_oracle(C, depth, W, H):
     out = render_gaussian_features(cam, *t, background=cu(bg), return_depth=depth)
     pre, f, ids, ranges, r = oracle_forward(cam, means, quats, scales, opac, colors=feats, bg=bg,
                                             depth=depth)
-    nc = r["n_contrib"]
+    nc, lists = r["n_contrib"], ranges[:, 1] - ranges[:, 0]
+    assert (lists.max() * lists.size >= 8 * lists.sum()) == crowd
     assert min(nc[0].max(), nc[-1].max(), nc[:, 0].max(), nc[:, -1].max()) > 0
     np.testing.assert_array_equal(host(out["n_contrib"]), nc)
     assert_bits(host(out["features"]), r["image"], "image")
@@ -163,6 +169,36 @@ def test_render_of_odd_frames_matches_oracle(C, depth, W, H):
     torch.autograd.backward([out["features"], out["alpha"]], [cu(g_img), cu(g_a)])
     g = oracle_backward(cam, means, quats, scales, opac, pre, f, ids, ranges, r, g_img, g_a, bg=bg)
     for name, a in zip(("means", "quats", "scales", "opacities", "features"), t):
-        # float32 sums against float32 terms summed in 64 bits, each over up to
-        # the frame's pixels: the repository's bound for these gradients
+        # the repository's bound for gradients of this chain (tests/test_gpu_parity.py)
         assert rel_err(host(a.grad), g[name]) < 1e-3, name
+
+
+@pytest.mark.parametrize("W,H", [(64, 64), (328, 200), (641, 359)])
+def test_order_holds_the_bands_lengths(W, H):
+    """Behind the order's T words: each band's longest list and its number of
+    entries, from the binning's placement and from the forward's own launch."""
+    from gpu_util import cu, host
+    from mlx3d_amd.cameras import Camera
+    from mlx3d_amd.splatting import render_gaussians
+    from mlx3d_amd.splatting.rasterize import raster_forward, tile_order_buffer
+
+    rng = np.random.default_rng(W)
+    n = 2000
+    cam = Camera.look_at(eye=(0.0, 0.0, -4.0), width=W, height=H)
+    t = [cu(np.asarray(a, np.float32)) for a in (
+        rng.standard_normal((n, 3)) * 0.7, rng.standard_normal((n, 4)),
+        rng.uniform(0.02, 0.1, (n, 3)), rng.uniform(0.1, 0.9, n), rng.random((n, 3)))]
+    t[0].requires_grad_(True)
+    out = render_gaussians(cam, *t[:4], colors=t[4])
+    placed = out["image"].grad_fn.saved_tensors[-1]  # the backward has not run
+    ranges, ids = out["tile_ranges"], out["sorted_ids"]
+    T = ranges.shape[0]
+    own = tile_order_buffer(W, H, ranges.device)
+    raster_forward(out["means2d"].detach(), cu(np.ones((n, 4), np.float32)), t[4], ids, ranges,
+                   None, W, H, tile_order=own)
+    lists = host(ranges[:, 1] - ranges[:, 0])
+    cuts = np.cumsum([0] + [T // 8 + (x < T % 8) for x in range(8)])
+    bands = [lists[a:b] for a, b in zip(cuts[:-1], cuts[1:])]
+    want = [b.max() for b in bands] + [b.sum() for b in bands]
+    for order in (placed, own):
+        np.testing.assert_array_equal(host(order)[2 * T:2 * T + 16], want)
