@@ -341,7 +341,9 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
 // 137, 512 -> 279; a box (300k) 82 -> 81, 79 -> 80, 103 -> 97; heavy tails (400k;
 // 1M at 32400) 38 -> 37, 69 -> 67, 126 -> 120, 432 -> 418; shells (1M), where
 // neighbouring tiles share the most, 85 -> 89, 104 -> 106, 178 -> 170, 457 -> 457;
-// 32 channels, 1M in a box at 8160 tiles, 451 -> 381.
+// 32 channels, 1M in a box at 8160 tiles, 451 -> 381.  Neighbouring tiles on
+// different XCDs cost traffic that the balance outweighs: 1M with SH at 1080p
+// reads and writes 181 MB instead of 91, of the 1.2 GB that fit in its time.
 __device__ __forceinline__ int tile_at(const int* order, uint32_t b, uint32_t nb, bool by_block) {
     if (!order) return (int)xcd_remap(b, nb);
     if (by_block) return order[b];
@@ -430,11 +432,11 @@ __device__ __forceinline__ float comp4(const float4& v, int e) {
 // for every pair of a wave and a Gaussian, and an LDS read costs two cycles
 // per register it fills, broadcast or not: a separate log-alpha bound, depth
 // and padded channels (12 registers) kept the LDS busy for 82 of the 91
-// million cycles in which a CU had work (1M Gaussians, 1080p), so a record
-// holds nothing the loop can do without.  Its 16-byte pieces lie in arrays of
-// their own, which a walk addresses by one offset of 16 x the staged index
-// (whole records of 32 to 96 bytes took up to six more registers and 0.5 to
-// 2 % longer, 16 channels 1 % less).
+// million cycles in which a CU had work (1M Gaussians, 1080p, 194 us), so a
+// record holds nothing the loop can do without (45 of 80 million, 157 us).  Its
+// 16-byte pieces lie in arrays of their own, which a walk addresses by one offset
+// of 16 x the staged index (whole records of 32 to 96 bytes took up to six more
+// registers and 0.5 to 2 % longer, 16 channels 1 % less).
 constexpr int kRecords = kThreads + 1;  // the last is the walk lists' padding
 template <int NV>
 struct FwdRec {
@@ -770,7 +772,7 @@ __global__ __launch_bounds__(kThreads, fwd_min_waves(CH)) void k_raster_fwd(GSX_
 // The forward of small frames.  One wave composites a quadrant's list serially
 // in k_raster_fwd, about 45 instructions an entry, and a wave alone on its
 // SIMD issues one every six cycles: the tile with the longest list bounds the
-// launch (2221 entries of a 256 x 256 view: 106 us, 87 us here).  Only the chain
+// launch (2221 entries of a 256 x 256 view: 106 us, 82 us here).  Only the chain
 // through T is serial, so here a workgroup has one quadrant: three waves evaluate
 // alphas, 16 entries of a chunk of 48 each, into LDS (zero where the pixel
 // does not take the entry), while wave 0 composites the chunk before.  The
@@ -1520,8 +1522,8 @@ constexpr int kMxGroup = 16;   // Gaussians per matrix-core group
 // 8.3, measured) with 12 to 20 waves on a compute unit.  Measured against the
 // kernels before it (pixels across the lanes with the sums on the VALU up to
 // 16 channels; the channel products through an LDS tile, geometric sums
-// through LDS atomics, at 32): 500k Gaussians, 32 channels, 720p 509 -> 285
-// us; 60k, 12 channels, 641 x 479 182 -> 111 us; 200k surfels, 5 channels,
+// through LDS atomics, at 32): 500k Gaussians, 32 channels, 720p 509 -> 284
+// us; 60k, 12 channels, 641 x 479 182 -> 118 us; 200k surfels, 5 channels,
 // 960 x 540 224 -> 147 us (all with the geometric gradients in one record,
 // below).  With three channels it gains 5 % where Gaussians are small and
 // loses 18 % where they cover many tiles (every quadrant stages the list for
@@ -1779,7 +1781,7 @@ __device__ __forceinline__ void bwd_bucket(const BwdLds& L, int b0, int cnt, Bwd
             // entry's own term is never in them.  Taking it back out of an
             // inclusive sum leaves that sum's rounding, which 1 / (1 - alpha)
             // multiplies by up to 100 (three-entry stacks with an opaque one:
-            // 5.7e-6 of the gradient's terms off, 2e-7 this way; 282 -> 286 us
+            // 5.7e-6 of the gradient's terms off, 2e-7 this way; 283 -> 284 us
             // at 32 channels, 500k, 720p).
             float Qa = lane_below(xa), Qb = lane_below(xb);
             row_scan_add(Qa, Qb);
@@ -1888,9 +1890,9 @@ __device__ __forceinline__ void bwd_bucket(const BwdLds& L, int b0, int cnt, Bwd
 }
 
 // The atomics of the bucket whose gradients lie in LDS.  An instruction's lanes
-// take whole entries, component by component: the atomics execute at 20.4 G
-// 64-byte lines/s whatever a line holds (measured, random and neighbouring
-// lines alike), so an entry's components go out together and lie in as few
+// take whole entries, component by component: the atomics execute at 20 to 21 G
+// 64-byte lines/s whatever a line holds (measured over 2 to 256 MiB, 4 to 16
+// floats of a line), so an entry's components go out together and lie in as few
 // lines as possible.  Memory operations complete in order, and a load issued
 // behind atomics waits for them too: the caller sends a bucket's gradients
 // once the loads of the next bucket have arrived, so that they drain under
@@ -1937,7 +1939,7 @@ constexpr int bwd_wide_waves(int chp) { return chp == 8 ? 5 : (chp == 16 ? 4 : 3
 // tile's four quadrants (1.06 with 1M Gaussians at 1080p), so summing the
 // quadrants' gradients before the atomics would save little, while batches
 // shared by the four waves cost four barriers each and leave 16 % of the
-// bucket lanes empty (32 channels: 367 us, against 283 us).
+// bucket lanes empty (32 channels: 367 us, against 283).
 template <int CHP>
 __global__ __launch_bounds__(kWave, bwd_wide_waves(CHP)) void k_raster_bwd_wide(
     const float2* __restrict__ xy, const float4* __restrict__ co, const float* __restrict__ feat,
