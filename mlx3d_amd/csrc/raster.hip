@@ -1940,6 +1940,12 @@ constexpr int bwd_wide_waves(int chp) { return chp == 8 ? 5 : (chp == 16 ? 4 : 3
 // quadrants' gradients before the atomics would save little, while batches
 // shared by the four waves cost four barriers each and leave 16 % of the
 // bucket lanes empty (32 channels: 367 us, against 283).
+//
+// A Gaussian's sums take up to four float atomics per tile this way.  That shows
+// where a few Gaussians cover the frame and carry the norm: 60k on shells at 641
+// x 479, 12 channels, one view of six, feature gradients 0.8e-6 -> 1.8e-6 off
+// 64 bits and opacities 0.7e-6 -> 1.0e-6; elsewhere (5 to 32 channels, surfels)
+// the errors are 0.7 to 1.1 times those of one atomic per tile.
 template <int CHP>
 __global__ __launch_bounds__(kWave, bwd_wide_waves(CHP)) void k_raster_bwd_wide(
     const float2* __restrict__ xy, const float4* __restrict__ co, const float* __restrict__ feat,
