@@ -1941,11 +1941,12 @@ constexpr int bwd_wide_waves(int chp) { return chp == 8 ? 5 : (chp == 16 ? 4 : 3
 // shared by the four waves cost four barriers each and leave 16 % of the
 // bucket lanes empty (32 channels: 367 us, against 283).
 //
-// A Gaussian's sums take up to four float atomics per tile this way.  That shows
-// where a few Gaussians cover the frame and carry the norm: 60k on shells at 641
-// x 479, 12 channels, one view of six, feature gradients 0.8e-6 -> 1.8e-6 off
-// 64 bits and opacities 0.7e-6 -> 1.0e-6; elsewhere (5 to 32 channels, surfels)
-// the errors are 0.7 to 1.1 times those of one atomic per tile.
+// A Gaussian's sums take up to four float atomics per tile this way, a few more
+// float32 steps for those that cover many tiles.  Against 64 bits, 48 passes of
+// 8 and 16 channels over four scenes: 1.03 to 1.06 times the error of one atomic
+// per tile in the mean; the most where a few large Gaussians carry the norm
+// (scales 0.8e-6 -> 2.6e-6, quaternions 3.2e-6 -> 7.5e-6, features 0.8e-6 ->
+// 1.8e-6); surfels and 32 channels as before.
 template <int CHP>
 __global__ __launch_bounds__(kWave, bwd_wide_waves(CHP)) void k_raster_bwd_wide(
     const float2* __restrict__ xy, const float4* __restrict__ co, const float* __restrict__ feat,
